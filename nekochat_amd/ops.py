@@ -140,7 +140,8 @@ def _issue(ctx: Context, fn, *args):
 def prepare(op, *args, **kwargs):
     """Validates op(*args, **kwargs) once and returns (run, result): run() re-issues the same C call
     on the same buffers with no Python-side checks -- for tight loops that replay one op. The stream
-    is the torch stream current at preparation time."""
+    is the torch stream current at preparation time. run() keeps the tensors it was given, and the
+    result, alive: the C call holds bare addresses."""
     _recording.rec = rec = []
     try:
         result = op(*args, **kwargs)
@@ -159,6 +160,7 @@ def prepare(op, *args, **kwargs):
         if rc != NEKO_OK:
             raise NekoError(lib.neko_hip_last_error(handle).decode(), rc)
 
+    run.held = (args, kwargs, result)
     return run, result
 
 

@@ -5,6 +5,8 @@ oracle (in practice almost every output is bit-identical: the kernels accumulate
 where the reference rounds). Configured shapes run at full size; edge cases cover empty inputs, odd
 widths (fallback kernels), strided rows, in-place calls, f32 activations and out-of-range positions.
 """
+import weakref
+
 import numpy as np
 import pytest
 import torch
@@ -70,6 +72,24 @@ def test_rmsnorm_strided_inplace_and_edges(dev):
     assert np.array_equal(to_bits(buf[:, C:]), tail), "columns past C were written"
     empty = torch.empty((0, C), dtype=torch.float16, device=dev)
     assert ops.rms_norm(empty, w, 1e-6).shape == (0, C)
+
+
+def test_prepared_call_keeps_its_buffers(dev):
+    """A prepared call holds addresses, so it keeps the tensors alive: dropped by the caller, their memory
+    is not given to the next allocation while the call exists, and is once it is gone."""
+    _case("prepared silu_mul keeps its buffers")
+    h = _f16((64, 512), 3, dev)
+    ref = weakref.ref(h)
+    run, out = ops.prepare(ops.silu_mul, h)
+    want = ops.silu_mul(h).clone()
+    del h
+    assert ref() is not None
+    torch.full((64, 512), 9.0, dtype=torch.float16, device=dev)  # would land on the freed input
+    run()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    del run
+    assert ref() is None
 
 
 def test_prepared_call_keeps_its_stream(dev):
