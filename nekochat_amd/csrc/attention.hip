@@ -3,6 +3,9 @@
 // for token t at position pos0 + t and query head h, out = sum_j softmax_j(scale * q_h . k_j) v_j over
 // cache rows j <= pos0 + t, k_j / v_j being kv head h / (n_head / n_kv) of those rows.
 //
+// Calls with enough work take the matrix cores where the head size is 64 or 128 (attention_mfma.hip); what
+// follows is the vector path for the rest.
+//
 // A workgroup of four waves per work item (token, kv head, block of up to four of the query heads that
 // share it, split of the keys), the item's steps of keys dealt round robin to its waves. Lane = (key
 // residue, 16-byte chunk of the head): each load instruction reads whole K or V head rows (16 lanes per
@@ -19,7 +22,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "internal.h"
+#include "attention.h"
 
 namespace neko_hip {
 namespace {
@@ -27,56 +30,12 @@ namespace {
 constexpr int kAttnHeads = 4;              // query heads per work item, at most (HB = 4 or 1)
 constexpr int kAttnWaves = 4;              // waves per work item (its steps interleaved)
 constexpr int64_t kAttnTargetWaves = 4096;  // keys split until a launch holds about this many waves
-constexpr int64_t kAttnMaxSplits = 1024;    // the merge kernel's LDS weights
 constexpr int64_t kAttnOneHeadBytes = int64_t{32} << 20;  // K + V bytes up to which items take one head
-
-struct AttnArgs {
-    const void* q;
-    int64_t qs;  // q row stride (elements)
-    const uint16_t* kc;
-    const uint16_t* vc;
-    int64_t kvw;  // cache row width (halves) = n_kv * hd
-    void* out;
-    int64_t os;  // out row stride (elements)
-    int64_t T;
-    int64_t pos0;
-    int n_head;
-    int n_kv;
-    int group;    // n_head / n_kv
-    int hblocks;  // ceil(group / HB): the head blocks per kv head
-    int hd;
-    float scale;
-    int splits;          // key splits per (token, kv head, head block)
-    int64_t split_keys;  // keys per split, a multiple of the kernel's step
-    float* part;         // splits > 1: [T][n_head][splits][hd + 2] = (max, sum, accumulators)
-};
 
 __device__ __forceinline__ void wave_sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ float readlane_f32(float v, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
-
-// Maximum / sum over the wave, returned wave-uniform (16-lane DPP all-reduce, then the four row results
-// combined in a fixed order). All 64 lanes active.
-__device__ __forceinline__ float wave_max_f32(float v) {
-    v = fmaxf(v, dpp_f32<kDppQuadXor1>(v));
-    v = fmaxf(v, dpp_f32<kDppQuadXor2>(v));
-    v = fmaxf(v, dpp_f32<kDppRowHalfMirror>(v));
-    v = fmaxf(v, dpp_f32<kDppRowMirror>(v));
-    return fmaxf(fmaxf(readlane_f32(v, 0), readlane_f32(v, 16)), fmaxf(readlane_f32(v, 32), readlane_f32(v, 48)));
-}
-
-__device__ __forceinline__ float wave_sum_f32(float v) {
-    v = v + dpp_f32<kDppQuadXor1>(v);
-    v = v + dpp_f32<kDppQuadXor2>(v);
-    v = v + dpp_f32<kDppRowHalfMirror>(v);
-    v = v + dpp_f32<kDppRowMirror>(v);
-    return (readlane_f32(v, 0) + readlane_f32(v, 16)) + (readlane_f32(v, 32) + readlane_f32(v, 48));
 }
 
 // Eight halves of a cache row at p -- dimensions d .. d + 7 of a head, those at or past hd read as 0 --
@@ -111,15 +70,6 @@ __device__ __forceinline__ float group_sum_f32(float v) {
     if constexpr (DC >= 16) v = v + dpp_f32<kDppRowMirror>(v);
     if constexpr (DC >= 32) v = v + __shfl_xor(v, 16);
     return v;
-}
-
-// Partial results of a key split (splits > 1): the accumulators [T][n_head][splits][hd] at part, then
-// (max, sum) pairs [T][n_head][splits][2] after them.
-__device__ __forceinline__ float* part_acc(const AttnArgs& a, int64_t th, int split) {
-    return a.part + (th * a.splits + split) * a.hd;
-}
-__device__ __forceinline__ float* part_ml(const AttnArgs& a, int64_t th, int split) {
-    return a.part + a.T * a.n_head * a.splits * a.hd + (th * a.splits + split) * 2;
 }
 
 // Lane layout: lane = (key residue r, chunk c) -- 16-byte chunk c (dimensions 8c .. 8c + 7) of key
@@ -331,7 +281,7 @@ __global__ __launch_bounds__(64 * NW) void attn_kernel(AttnArgs a) {
 // Merges the key splits of one (token, head) per workgroup of 256 threads: M = the largest split
 // maximum, each split weighted by exp(max - M); the sums and the accumulators added over the splits
 // (threads over splits and dimensions, then the waves and groups in a fixed order); out = acc / sum.
-template <typename TQ>
+template <typename TQ, bool LOG2>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
     constexpr int kPer = kAttnMaxSplits / 256;  // splits per thread, at most
     __shared__ float wsh[kAttnMaxSplits];
@@ -361,7 +311,8 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
         const int s = tid + 256 * k;
-        const float ws = expf(ms[k] - mx);  // an empty split or none: exp(-inf) = 0
+        // An empty split or none: exp(-inf) = 0.
+        const float ws = LOG2 ? __builtin_amdgcn_exp2f(ms[k] - mx) : expf(ms[k] - mx);
         if (s < S) wsh[s] = ws;
         sum = __builtin_fmaf(ws, ls[k], sum);
     }
@@ -414,9 +365,7 @@ int launch_hdp(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool vec,
     if (one_head) launch_hb<TQ, HDP, 1>(ctx, a, grid, vec, pf);
     else launch_hb<TQ, HDP, kAttnHeads>(ctx, a, grid, vec, pf);
     if (int rc = after_launch(ctx, what)) return rc;
-    if (a.splits == 1) return NEKO_OK;
-    hipLaunchKernelGGL((attn_merge_kernel<TQ>), dim3(static_cast<uint32_t>(a.T * a.n_head)), dim3(256), 0, ctx->stream, a);
-    return after_launch(ctx, what);
+    return a.splits == 1 ? NEKO_OK : attn_merge(ctx, what, a, sizeof(TQ) == 2 ? NEKO_DT_F16 : NEKO_DT_F32, false);
 }
 
 template <typename TQ>
@@ -427,6 +376,19 @@ int launch_typed(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool ve
 }
 
 }  // namespace
+
+int attn_merge(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, int dtype, bool log2) {
+    const dim3 grid(static_cast<uint32_t>(a.T * a.n_head)), block(256);
+    if (dtype == NEKO_DT_F16) {
+        if (log2) hipLaunchKernelGGL((attn_merge_kernel<half_t, true>), grid, block, 0, ctx->stream, a);
+        else hipLaunchKernelGGL((attn_merge_kernel<half_t, false>), grid, block, 0, ctx->stream, a);
+    } else {
+        if (log2) hipLaunchKernelGGL((attn_merge_kernel<float, true>), grid, block, 0, ctx->stream, a);
+        else hipLaunchKernelGGL((attn_merge_kernel<float, false>), grid, block, 0, ctx->stream, a);
+    }
+    return after_launch(ctx, what);
+}
+
 }  // namespace neko_hip
 
 using namespace neko_hip;
@@ -500,6 +462,7 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
         if (int rc = workspace(ctx, bytes, &ws)) return rc;
         a.part = static_cast<float*>(ws);
     }
+    if (attn_mfma_takes(a)) return attn_mfma(ctx, what, a, dtype);
     const bool vec = hd % 8 == 0 && aligned(k_cache, 16) && aligned(v_cache, 16);
     return dtype == NEKO_DT_F16 ? launch_typed<half_t>(ctx, what, a, vec, items, one_head)
                                 : launch_typed<float>(ctx, what, a, vec, items, one_head);

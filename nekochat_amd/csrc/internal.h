@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <string>
@@ -76,6 +77,11 @@ int capturing(neko_hip_ctx* ctx, hipStream_t stream, bool* yes);
 // grid of a persistent kernel: that many per CU, or fewer when there is less work.
 int resident_blocks_per_cu(const void* kernel, int block, size_t lds_bytes = 0);
 int64_t persistent_grid(neko_hip_ctx* ctx, const void* kernel, int block, int64_t work_blocks, size_t lds_bytes = 0);
+
+// Kernels taking more than 64 KB of dynamic LDS must be allowed it per device (hipFuncSetAttribute on
+// the context's device, which enter() made current); `done` records which devices have been, one bit
+// per device id, safely across host threads.
+int allow_lds(neko_hip_ctx* ctx, const void* kernel, size_t bytes, std::atomic<uint64_t>& done);
 
 // The KV-cache store's launch (kv_store.hip), after argument checks; also the second half of the
 // unfused q/k RoPE + KV store path.

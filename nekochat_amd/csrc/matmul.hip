@@ -29,18 +29,6 @@ namespace {
 
 constexpr int kBlockK = 32;  // quant.h kQuantBlock
 
-// Kernels taking more than 64 KB of dynamic LDS must be allowed it per device (hipFuncSetAttribute on
-// the context's device, which enter() made current); `done` records which devices have been, one bit
-// per device id, safely across host threads.
-int allow_lds(neko_hip_ctx* ctx, const void* kernel, size_t bytes, std::atomic<uint64_t>& done) {
-    const uint64_t bit = uint64_t(1) << (ctx->device & 63);
-    if (done.load(std::memory_order_acquire) & bit) return NEKO_OK;
-    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
-    if (e != hipSuccess) return fail(ctx, NEKO_ERR_HIP, "matmul: hipFuncSetAttribute: %s", hipGetErrorString(e));
-    done.fetch_or(bit, std::memory_order_release);
-    return NEKO_OK;
-}
-
 struct MmArgs {
     const void* x;
     int64_t xs;

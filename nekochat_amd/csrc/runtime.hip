@@ -111,6 +111,15 @@ int workspace(neko_hip_ctx* ctx, size_t bytes, void** out, int slot) {
     return NEKO_OK;
 }
 
+int allow_lds(neko_hip_ctx* ctx, const void* kernel, size_t bytes, std::atomic<uint64_t>& done) {
+    const uint64_t bit = uint64_t(1) << (ctx->device & 63);
+    if (done.load(std::memory_order_acquire) & bit) return NEKO_OK;
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    if (e != hipSuccess) return fail(ctx, NEKO_ERR_HIP, "hipFuncSetAttribute (dynamic LDS): %s", hipGetErrorString(e));
+    done.fetch_or(bit, std::memory_order_release);
+    return NEKO_OK;
+}
+
 }  // namespace neko_hip
 
 using namespace neko_hip;

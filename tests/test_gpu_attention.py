@@ -128,6 +128,64 @@ def test_attention_scale_and_single_key(dev):
         assert torch.allclose(out[t].double().cpu(), want, rtol=0, atol=1e-5)
 
 
+# Rows = tokens x query heads per kv head, 32 to a wave: one, two or four row groups per workgroup and
+# key tiles of 128 or 64, at their edges, split over the keys and not.
+@pytest.mark.parametrize("T,H,KV,hd,pos0", [
+    (8, 8, 2, 128, 119),     # 32 rows, 127 keys: the last row group and key tile short of one
+    (8, 8, 2, 64, 121),      # 129 keys: one past a tile
+    (16, 8, 2, 128, 48),     # 64 rows, 64 keys
+    (17, 8, 2, 128, 0),      # 68 rows: four row groups, the last two empty but for 4 rows
+    (32, 8, 2, 64, 33),      # 128 rows, 65 keys
+    (33, 8, 2, 128, 640),    # 132 rows: a second row tile of 4 rows, keys split
+    (43, 6, 2, 128, 515),    # three heads per kv head: tokens straddle waves and row tiles
+    (129, 3, 3, 64, 0),      # one head per kv head
+    (300, 16, 1, 128, 1),    # sixteen heads per kv head, splits empty for the first rows
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_attention_row_and_key_tiles(dev, T, H, KV, hd, pos0, dtype):
+    """q rows of very different sizes (each is scaled by its own power of two). The scores' f32 rounding
+    weighs on the weights by its absolute size, so q is kept to scores of a few units and the bar is
+    the one above; f16 outputs as in test_attention_f16."""
+    _case(f"attention tiles T={T} H={H} KV={KV} hd={hd} pos0={pos0} {dtype}")
+    q, kc, vc = _inputs(T, H, KV, hd, pos0, dev, seed=T + hd)
+    q *= 2.0 ** torch.randint(-12, 1, (T, 1), generator=torch.Generator().manual_seed(1)).to(dev)
+    q = q.to(dtype)
+    out = ops.attention(q, kc, vc, H, KV, hd, pos0)
+    torch.cuda.synchronize()
+    want = _oracle(q, kc, vc, H, KV, hd, pos0)
+    half_ulp = 0 if dtype == torch.float32 else np.spacing(np.abs(want).astype(np.float16)).astype(np.float32) / 2
+    excess = np.abs(out.float().cpu().numpy() - want) - half_ulp - TOL * (1.0 + np.abs(want))
+    print(f"worst excess {excess.max():.3e}", flush=True)
+    assert (excess <= 0).all()
+
+
+@pytest.mark.parametrize("T,pos0", [(3, 200), (12, 200), (40, 70), (40, 900)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_attention_infinities(dev, T, pos0, dtype):
+    """A key of score -inf weighs nothing; an infinite or NaN v row reaches the tokens that see it and no
+    earlier one, and a negative scale turns the scores round: as the oracle has it."""
+    _case(f"attention infinities T={T} pos0={pos0} {dtype}")
+    H, KV, hd = 8, 2, 128
+    q, kc, vc = _inputs(T, H, KV, hd, pos0, dev, seed=T + pos0)
+    q = q.abs().to(dtype)
+    kc[5] = -float("inf")
+    vc[pos0 + T // 2, 3] = float("nan")
+    vc[pos0 + T - 1, 7] = float("inf")
+    out = ops.attention(q, kc, vc, H, KV, hd, pos0)
+    torch.cuda.synchronize()
+    want, got = _oracle(q, kc, vc, H, KV, hd, pos0), out.float().cpu().numpy()
+    assert np.isfinite(want[0, hd:]).all() and np.isnan(want[-1, 3])
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    bar = 5e-4 if dtype == torch.float16 else TOL  # an f16 rounding: 2^-11
+    assert (np.abs(got - want)[ok] <= bar * (1 + np.abs(want[ok]))).all()
+    kc[5] = 1.0
+    vc = torch.nan_to_num(vc, nan=0.0, posinf=0.0)
+    a = ops.attention(q, kc, vc, H, KV, hd, pos0, scale=-0.1)
+    b = ops.attention(-q, kc, vc, H, KV, hd, pos0, scale=0.1)
+    assert torch.equal(a, b)
+
+
 def test_attention_argument_checks(dev):
     _case("attention argument checks")
     q, kc, vc = _inputs(2, 4, 2, 64, 5, dev, seed=5)
