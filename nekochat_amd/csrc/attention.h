@@ -63,7 +63,7 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 // Combines the splits of a.part into a.out (log2: the maxima are base-2 exponents).
 int attn_merge(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, int dtype, bool log2);
 // The matrix-core path (attention_mfma.hip): whether it takes this call, and its launches, where it does.
-bool attn_mfma_takes(const AttnArgs& a);
+bool attn_mfma_takes(const AttnArgs& a, int dtype);
 int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype);
 
 }  // namespace neko_hip

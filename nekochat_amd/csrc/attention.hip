@@ -29,6 +29,7 @@ namespace {
 
 constexpr int kAttnHeads = 4;              // query heads per work item, at most (HB = 4 or 1)
 constexpr int kAttnWaves = 4;              // waves per work item (its steps interleaved)
+constexpr int kAttnWideWaves = 8;                // the same where one workgroup then takes a head's whole row
 constexpr int64_t kAttnTargetWaves = 4096;  // keys split until a launch holds about this many waves
 constexpr int64_t kAttnOneHeadBytes = int64_t{32} << 20;  // K + V bytes up to which items take one head
 
@@ -355,8 +356,15 @@ void launch_hb(neko_hip_ctx* ctx, const AttnArgs& a, dim3 grid, bool vec, bool p
 }
 
 template <typename TQ, int HDP>
-int launch_hdp(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool vec, int64_t items, bool one_head) {
+int launch_hdp(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool vec, int64_t items, bool one_head, bool wide) {
     const dim3 grid(static_cast<uint32_t>(items));
+    if constexpr (HDP <= 128) {  // (wider heads spill in the 128 registers of such a workgroup's lanes)
+        if (wide) {
+            hipLaunchKernelGGL((attn_kernel<TQ, HDP, true, kAttnWideWaves, 1, false>), grid, dim3(64 * kAttnWideWaves), 0,
+                               ctx->stream, a);
+            return after_launch(ctx, what);
+        }
+    }
     // The prefetching form where a wave has more than one step (measured: 4096-position decode, one
     // step per wave, 12.7 us without and 15.5 with it; 32768 positions 56.3 -> 49.6 us, the 2048- and
     // 8192-token prefills 6% faster).
@@ -369,10 +377,10 @@ int launch_hdp(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool vec,
 }
 
 template <typename TQ>
-int launch_typed(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool vec, int64_t items, bool one_head) {
-    if (a.hd <= 64) return launch_hdp<TQ, 64>(ctx, what, a, vec, items, one_head);
-    if (a.hd <= 128) return launch_hdp<TQ, 128>(ctx, what, a, vec, items, one_head);
-    return launch_hdp<TQ, 256>(ctx, what, a, vec, items, one_head);
+int launch_typed(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool vec, int64_t items, bool one_head, bool wide) {
+    if (a.hd <= 64) return launch_hdp<TQ, 64>(ctx, what, a, vec, items, one_head, wide);
+    if (a.hd <= 128) return launch_hdp<TQ, 128>(ctx, what, a, vec, items, one_head, wide);
+    return launch_hdp<TQ, 256>(ctx, what, a, vec, items, one_head, wide);
 }
 
 }  // namespace
@@ -452,6 +460,13 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
         const int64_t want = (kAttnTargetWaves + base * kAttnWaves - 1) / (base * kAttnWaves);
         splits = std::min<int64_t>({want, (steps + kAttnWaves - 1) / kAttnWaves, kAttnMaxSplits});
     }
+    const bool vec = hd % 8 == 0 && aligned(k_cache, 16) && aligned(v_cache, 16);
+    // Eight waves on a head's whole row instead of splits and their merge, while each wave has one step and
+    // the launch's workgroups fit at once (two per CU): one token over 201 keys, 32 / 8 heads of 128, f16,
+    // 8.3 us split and 6.2 whole, over 501 keys, 12 heads of 64, 8.5 and 5.8. At two steps there is
+    // nothing left of that (16 waves of one step or 8 of two over 501 keys of 128: 8.6 and 8.5).
+    const bool wide = vec && hd <= 128 && one_head && splits > 1 && steps <= kAttnWideWaves && base <= 2 * ctx->cu_count;
+    if (wide) splits = 1;
     a.split_keys = (steps + splits - 1) / splits * step;
     a.splits = static_cast<int>((keys + a.split_keys - 1) / a.split_keys);
     const int64_t items = base * a.splits;
@@ -462,8 +477,7 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
         if (int rc = workspace(ctx, bytes, &ws)) return rc;
         a.part = static_cast<float*>(ws);
     }
-    if (attn_mfma_takes(a)) return attn_mfma(ctx, what, a, dtype);
-    const bool vec = hd % 8 == 0 && aligned(k_cache, 16) && aligned(v_cache, 16);
-    return dtype == NEKO_DT_F16 ? launch_typed<half_t>(ctx, what, a, vec, items, one_head)
-                                : launch_typed<float>(ctx, what, a, vec, items, one_head);
+    if (attn_mfma_takes(a, dtype)) return attn_mfma(ctx, what, a, dtype);
+    return dtype == NEKO_DT_F16 ? launch_typed<half_t>(ctx, what, a, vec, items, one_head, wide)
+                                : launch_typed<float>(ctx, what, a, vec, items, one_head, wide);
 }

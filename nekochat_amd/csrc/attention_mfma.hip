@@ -33,7 +33,7 @@ namespace {
 
 constexpr int kRaise = 8;    // the maximum is raised when a score exceeds it by more (in log2)
 constexpr int kOffset = 6;   // probabilities are held times 2^kOffset: <= 2^14, within f16
-constexpr double kMinWork = 70000, kMinPromptWork = 28000, kPromptRows = 100;  // see attn_mfma_takes
+constexpr double kMinWorkF16 = 70000, kMinWorkF32 = 112000, kMinPromptWork = 28000, kPromptRows = 100;  // see attn_mfma_takes
 constexpr float kNoKey = -1e30f;  // the running maximum before the first key
 
 typedef short short4v __attribute__((ext_vector_type(4)));
@@ -497,19 +497,20 @@ int launch_rows(neko_hip_ctx* ctx, const AttnArgs& a, int rw, int row_tiles, boo
 
 }  // namespace
 
-bool attn_mfma_takes(const AttnArgs& a) {
+bool attn_mfma_takes(const AttnArgs& a, int dtype) {
     // 32-bit row numbers and offsets within a tile; whole 16-byte chunks.
     if ((a.hd != 64 && a.hd != 128) || !aligned(a.kc, 16) || !aligned(a.vc, 16) || a.kvw > (1 << 20) ||
         a.T * a.group >= (int64_t{1} << 31) - 256)
         return false;
-    // From kMinWork query-head x key pairs of 128 dimensions; below, the vector path's shorter start wins:
+    // From kMinWorkF16 / F32 query-head x key pairs of 128 dimensions; below, the vector path's shorter start wins:
     // with 32 / 8 heads of 128, f16, 4 tokens over 504 keys (64 k pairs) take 11.0 us there and 11.6 here, 2
     // over 1502 (96 k) 12.9 and 11.7, 1 over 4001 (128 k) 13.5 and 11.0, 8 over 508 (130 k) 12.9 and
-    // 10.4. Prompts, whose rows fill the columns of several waves, from kMinPromptWork: 100 tokens
+    // 10.4; f32, 12 tokens of 16 / 8 heads over 512 keys (97 k) 12.2 and 14.2, 1 of 32 / 8 over 4001 (128 k)
+    // 13.5 and 11.5. Prompts, whose rows fill the columns of several waves, from kMinPromptWork: 100 tokens
     // from 0, 12 heads of 64 (30 k) 11.5 and 7.0.
     const double rows = static_cast<double>(a.T) * a.group;
     const double work = rows * a.n_kv * static_cast<double>(a.pos0 + (a.T + 1) / 2) / (128 / a.hd);
-    return work >= (rows >= kPromptRows ? kMinPromptWork : kMinWork);
+    return work >= (rows >= kPromptRows ? kMinPromptWork : dtype == NEKO_DT_F16 ? kMinWorkF16 : kMinWorkF32);
 }
 
 int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype) {

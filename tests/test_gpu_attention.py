@@ -128,18 +128,23 @@ def test_attention_scale_and_single_key(dev):
         assert torch.allclose(out[t].double().cpu(), want, rtol=0, atol=1e-5)
 
 
-# Rows = tokens x query heads per kv head, 32 to a wave: one, two or four row groups per workgroup and
-# key tiles of 128 or 64, at their edges, split over the keys and not.
+# The matrix-core path (rows = tokens x query heads per kv head, 32 to a wave): one, two or four row groups
+# per workgroup and key tiles of 128 or 64, at their edges, split over the keys and not; then short rows.
 @pytest.mark.parametrize("T,H,KV,hd,pos0", [
-    (8, 8, 2, 128, 119),     # 32 rows, 127 keys: the last row group and key tile short of one
-    (8, 8, 2, 64, 121),      # 129 keys: one past a tile
-    (16, 8, 2, 128, 48),     # 64 rows, 64 keys
-    (17, 8, 2, 128, 0),      # 68 rows: four row groups, the last two empty but for 4 rows
-    (32, 8, 2, 64, 33),      # 128 rows, 65 keys
-    (33, 8, 2, 128, 640),    # 132 rows: a second row tile of 4 rows, keys split
+    (8, 128, 32, 128, 119),  # 32 rows, 127 keys: one row group, the key tile short of one
+    (8, 256, 64, 64, 121),   # 129 keys: one past a tile
+    (16, 128, 32, 128, 48),  # 64 rows, 64 keys: two row groups
+    (17, 64, 16, 128, 100),  # 68 rows: four row groups, the third with 4 rows, the last empty
+    (32, 64, 16, 64, 33),    # 128 rows, 65 keys
+    (33, 16, 4, 128, 640),   # 132 rows: a second row tile of 4 rows, keys split
     (43, 6, 2, 128, 515),    # three heads per kv head: tokens straddle waves and row tiles
-    (129, 3, 3, 64, 0),      # one head per kv head
+    (129, 12, 12, 64, 0),    # one head per kv head
     (300, 16, 1, 128, 1),    # sixteen heads per kv head, splits empty for the first rows
+    (1, 8, 2, 128, 128),     # below: a head's whole row by eight waves; 129 keys, five waves with a step
+    (2, 8, 2, 128, 254),     # 256 keys: every wave's step full
+    (1, 8, 2, 128, 256),     # 257 keys: split again
+    (1, 6, 6, 64, 511),      # 512 keys of 64 dimensions
+    (3, 4, 2, 40, 400),      # dimensions past 40 masked
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_attention_row_and_key_tiles(dev, T, H, KV, hd, pos0, dtype):
@@ -159,7 +164,7 @@ def test_attention_row_and_key_tiles(dev, T, H, KV, hd, pos0, dtype):
     assert (excess <= 0).all()
 
 
-@pytest.mark.parametrize("T,pos0", [(3, 200), (12, 200), (40, 70), (40, 900)])
+@pytest.mark.parametrize("T,pos0", [(3, 200), (2, 9000), (12, 2000), (40, 75), (40, 900)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_attention_infinities(dev, T, pos0, dtype):
     """A key of score -inf weighs nothing; an infinite or NaN v row reaches the tokens that see it and no
