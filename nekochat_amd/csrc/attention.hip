@@ -440,6 +440,11 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
     a.n_head = n_head;
     a.n_kv = n_kv;
     a.group = n_head / n_kv;
+    a.hd = hd;
+    a.scale = scale;
+    NEKO_REQUIRE(ctx, T * n_head <= 0x7fffffff, "%s: grid too large", what);
+    // Before the vector path's plan, whose workspace these calls do not use.
+    if (attn_mfma_takes(a, dtype)) return attn_mfma(ctx, what, a, dtype);
     // One query head per item where the K and V rows are few (their re-reads by the group's heads stay
     // in L2) and the launch would otherwise be short of waves; else up to four heads share each load.
     const int64_t kv_bytes = (pos0 + T) * static_cast<int64_t>(n_kv) * hd * 4;
@@ -447,8 +452,6 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
                           kv_bytes <= kAttnOneHeadBytes;
     const int hb_size = one_head ? 1 : kAttnHeads;
     a.hblocks = (a.group + hb_size - 1) / hb_size;
-    a.hd = hd;
-    a.scale = scale;
     // Split the keys when tokens x kv heads x head blocks leave the chip short of waves (each split at
     // least one 64-key step per wave).
     const int64_t base = T * n_kv * a.hblocks;
@@ -470,14 +473,13 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
     a.split_keys = (steps + splits - 1) / splits * step;
     a.splits = static_cast<int>((keys + a.split_keys - 1) / a.split_keys);
     const int64_t items = base * a.splits;
-    NEKO_REQUIRE(ctx, items <= 0x7fffffff && T * n_head <= 0x7fffffff, "%s: grid too large", what);
+    NEKO_REQUIRE(ctx, items <= 0x7fffffff, "%s: grid too large", what);
     if (a.splits > 1) {
         void* ws = nullptr;
         const size_t bytes = static_cast<size_t>(T) * n_head * a.splits * (hd + 2) * sizeof(float);
         if (int rc = workspace(ctx, bytes, &ws)) return rc;
         a.part = static_cast<float*>(ws);
     }
-    if (attn_mfma_takes(a, dtype)) return attn_mfma(ctx, what, a, dtype);
     return dtype == NEKO_DT_F16 ? launch_typed<half_t>(ctx, what, a, vec, items, one_head, wide)
                                 : launch_typed<float>(ctx, what, a, vec, items, one_head, wide);
 }

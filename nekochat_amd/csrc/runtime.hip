@@ -93,8 +93,8 @@ int workspace(neko_hip_ctx* ctx, size_t bytes, void** out, int slot) {
         if (int rc = capturing(ctx, ctx->stream, &cap)) return rc;
         if (cap)
             return fail(ctx, NEKO_ERR_INVALID,
-                        "matmul workspace must grow to %zu bytes (holds %zu) while the stream is being captured: make "
-                        "one uncaptured call at the largest shape first, or capture neko_hip_matmul_noalloc",
+                        "workspace must grow to %zu bytes (holds %zu) while the stream is being captured: make one "
+                        "uncaptured call at the largest shape first (a matmul: or capture neko_hip_matmul_noalloc)",
                         bytes, ctx->workspace_bytes[slot]);
         // The next power of two (at least 1 MiB): the buffers a slot outgrows add up to less than the
         // one it has, however the requests rise.

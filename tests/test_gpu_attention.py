@@ -191,6 +191,44 @@ def test_attention_infinities(dev, T, pos0, dtype):
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("T,H,KV,hd,pos0", [(1, 32, 8, 128, 4095), (70, 8, 2, 64, 900)])
+@pytest.mark.parametrize("warm", [False, True])
+def test_attention_captured(dev, T, H, KV, hd, pos0, warm):
+    """Under graph capture the workspace cannot grow: a fresh context's matrix-core call takes as many key
+    splits as fit (here one); after an eager call it takes the same splits. Replays follow their inputs."""
+    _case(f"attention captured T={T} H={H} KV={KV} hd={hd} pos0={pos0} warm={warm}")
+    from nekochat_amd._lib import lib
+    ctx = ops.Context(dev.index)
+    q, kc, vc = _inputs(T, H, KV, hd, pos0, dev, seed=T + pos0)
+    out, eager = torch.zeros_like(q), torch.zeros_like(q)
+    scale = 1.0 / hd ** 0.5
+
+    def call(o):
+        assert lib.neko_hip_set_stream(ctx.handle, torch.cuda.current_stream().cuda_stream or None) == 0
+        return lib.neko_hip_attention(ctx.handle, q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(), o.data_ptr(),
+                                      o.stride(0), T, H, KV, hd, pos0, scale, ops.DT_F32)
+
+    if warm:
+        assert call(eager) == 0
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        rc = call(out)
+    assert rc == 0, lib.neko_hip_last_error(ctx.handle).decode()
+    for k in range(3):
+        q.mul_(0.75)
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _check_f32(out, _oracle(q, kc, vc, H, KV, hd, pos0), f"replay {k}")
+        if warm:
+            assert call(eager) == 0
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager)
+    assert lib.neko_hip_set_stream(ctx.handle, None) == 0
+    ctx.close()
+
+
 def test_attention_argument_checks(dev):
     _case("attention argument checks")
     q, kc, vc = _inputs(2, 4, 2, 64, 5, dev, seed=5)
