@@ -20,6 +20,7 @@
 // workspace, and attn_merge_kernel combines them. The reference's CPU loop and its shader already sum
 // in different orders; any order here is one more within the same bound.
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 
 #include "attention.h"
@@ -162,7 +163,8 @@ __global__ __launch_bounds__(64 * NW) void attn_kernel(AttnArgs a) {
         for (int i = 0; i < HB; i++) {
             if (i >= nh) break;
             const float s = lane < STEP ? sw[i][lane] : -INFINITY;
-            const float mn = fmaxf(m[i], wave_max_f32(s));  // finite: the step holds a valid key
+            // Above -inf also where every score so far is -inf (or NaN): their weights are 0, not exp(-inf + inf).
+            const float mn = fmaxf(fmaxf(m[i], wave_max_f32(s)), -FLT_MAX);
             const float corr = expf(m[i] - mn);             // 0 on the wave's first step (m = -inf)
             const float p = expf(s - mn);                   // 0 for keys past k1
             l[i] = l[i] * corr + wave_sum_f32(p);
@@ -307,7 +309,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
     mx = wave_max_f32(mx);
     if ((tid & 63) == 0) red[0][wave] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));  // finite: split 0 holds key 0
+    mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));  // above -inf: split 0 holds key 0
     float sum = 0.0f;
 #pragma unroll
     for (int k = 0; k < kPer; k++) {

@@ -229,6 +229,29 @@ def test_attention_captured(dev, T, H, KV, hd, pos0, warm):
     ctx.close()
 
 
+@pytest.mark.parametrize("T,H,KV,hd,pos0,n", [
+    (1, 8, 2, 128, 200, 100),      # one workgroup per head: three waves see only such keys
+    (1, 8, 2, 96, 9000, 3000),     # whole splits
+    (300, 8, 2, 96, 0, 70),        # no splits: the first 70 tokens see nothing else
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("low", [-float("inf"), float("nan")])
+def test_attention_infinite_prefix(dev, T, H, KV, hd, pos0, n, dtype, low):
+    """The first n keys score -inf (weight 0, and NaN for a token that sees only such) or NaN, whole steps, waves
+    and splits of them: as the oracle has it."""
+    _case(f"attention infinite prefix T={T} H={H} KV={KV} hd={hd} pos0={pos0} n={n} {dtype} {low}")
+    q, kc, vc = _inputs(T, H, KV, hd, pos0, dev, seed=T + pos0)
+    q = q.abs().to(dtype)
+    kc[:n] = low
+    out = ops.attention(q, kc, vc, H, KV, hd, pos0)
+    torch.cuda.synchronize()
+    want, got = _oracle(q, kc, vc, H, KV, hd, pos0), out.float().cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = np.isfinite(want)
+    bar = 5e-4 if dtype == torch.float16 else TOL
+    assert (np.abs(got - want)[ok] <= bar * (1 + np.abs(want[ok]))).all()
+
+
 def test_attention_argument_checks(dev):
     _case("attention argument checks")
     q, kc, vc = _inputs(2, 4, 2, 64, 5, dev, seed=5)
