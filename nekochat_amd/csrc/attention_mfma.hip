@@ -16,7 +16,11 @@
 // f32. The running maximum is kept as an integer exponent, in which rescaling and merging are exact,
 // and raised only when a score exceeds it by 8.
 // Rows whose result is not finite (an infinity or NaN among the inputs may have met a zero weight or
-// the other plane of a split) are done again by attend_row, in the order of the definition.
+// the other plane of a split) are done again by the workgroup as the vector path's items (attend_item). Where
+// that takes every row a call costs more than the vector path alone would (one infinite v, f16; 32 / 8 heads of
+// 128: 8192 tokens 24.1 ms and 22.3, 2048 tokens 2.65 and 1.59, 1 over 32768 keys 70 us and 53; 12 heads of
+// 64, 1024 tokens, 570 and 215): a workgroup does its 128 rows one after the other and waits for each step's
+// loads. Loading ahead would take the registers of a second workgroup per CU from every call.
 //
 // What bounds it: the MFMAs -- the work counted twice in both products with f32 q, in one with f16 q -- with
 // the softmax's ~11 VALU operations per score beside them from the second wave of each SIMD. Measured
@@ -26,7 +30,7 @@
 #include <algorithm>
 #include <atomic>
 
-#include "attention.h"
+#include "attention_item.h"
 
 namespace neko_hip {
 namespace {
@@ -34,6 +38,7 @@ namespace {
 constexpr int kRaise = 8;    // the maximum is raised when a score exceeds it by more (in log2)
 constexpr int kOffset = 6;   // probabilities are held times 2^kOffset: <= 2^14, within f16
 constexpr double kMinWorkF16 = 70000, kMinWorkF32 = 112000, kMinPromptWork = 28000, kPromptRows = 100;  // see attn_mfma_takes
+constexpr int kRedoHeads = 4;     // query heads per item of the rows done again, at most
 constexpr float kNoKey = -1e30f;  // the running maximum before the first key
 
 typedef short short4v __attribute__((ext_vector_type(4)));
@@ -62,58 +67,6 @@ __device__ __forceinline__ float half_swap_sum(float v) {
     return __builtin_bit_cast(float, static_cast<uint32_t>(r[0])) + __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
 }
 
-// One row (token t, head h) over keys [k0, k1) by one wave, as the definition reads: scores with one lane
-// per key, streaming softmax, then lanes over the head's dimensions. For rows with infinities or NaN.
-template <typename TQ, int HD>
-__device__ __forceinline__ void attend_row(const AttnArgs& a, int64_t t, int g, int h, int64_t k0, int64_t k1, int split) {
-    const int lane = static_cast<int>(threadIdx.x) & 63;
-    constexpr int DPL = HD / 64;
-    const TQ* q = static_cast<const TQ*>(a.q) + t * a.qs + static_cast<int64_t>(h) * HD;
-    const half_t* kb = reinterpret_cast<const half_t*>(a.kc) + static_cast<int64_t>(g) * HD;
-    const half_t* vb = reinterpret_cast<const half_t*>(a.vc) + static_cast<int64_t>(g) * HD;
-    float m = -INFINITY, l = 0.0f, o[DPL] = {};
-#pragma unroll 1
-    for (int64_t j0 = k0; j0 < k1; j0 += 64) {
-        const int n = k1 - j0 < 64 ? static_cast<int>(k1 - j0) : 64;
-        float s = -INFINITY;
-        if (lane < n) {
-            const half_t* kr = kb + (j0 + lane) * a.kvw;
-            float p = 0.0f;
-#pragma unroll 1
-            for (int d = 0; d < HD; d += 8) {
-                const half8 k8 = *reinterpret_cast<const half8*>(kr + d);
-                for (int e = 0; e < 8; e++) p = __builtin_fmaf(to_f32(q[d + e]), to_f32(k8[e]), p);
-            }
-            s = p * a.scale;
-        }
-        const float mn = fmaxf(m, wave_max_f32(s));
-        const float corr = expf(m - mn);
-        const float p = lane < n ? expf(s - mn) : 0.0f;
-        l = l * corr + wave_sum_f32(p);
-        for (int e = 0; e < DPL; e++) o[e] *= corr;
-        m = mn;
-#pragma unroll 1
-        for (int j = 0; j < n; j++) {
-            const float w = readlane_f32(p, j);
-            const half_t* vr = vb + (j0 + j) * a.kvw + lane * DPL;
-            for (int e = 0; e < DPL; e++) o[e] = __builtin_fmaf(w, to_f32(vr[e]), o[e]);
-        }
-    }
-    if (a.splits == 1) {
-        TQ* orow = static_cast<TQ*>(a.out) + t * a.os + static_cast<int64_t>(h) * HD + lane * DPL;
-        const float inv = 1.0f / l;
-        for (int e = 0; e < DPL; e++) orow[e] = from_f32<TQ>(o[e] * inv);
-    } else {
-        float* pa = part_acc(a, t * a.n_head + h, split) + lane * DPL;
-        for (int e = 0; e < DPL; e++) pa[e] = o[e];
-        if (lane == 0) {
-            float* pm = part_ml(a, t * a.n_head + h, split);
-            pm[0] = m * 1.44269504088896341f;  // the merge works in log2
-            pm[1] = l;
-        }
-    }
-}
-
 // Four row groups at most: RW row groups of 32 rows x KW waves that share a group, each taking 32 KB_ of
 // the tile's keys.
 template <int HD, int RW, int KW, int KB_>
@@ -137,7 +90,7 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
     constexpr int NC = !kTwo ? 1 : KW > 1 ? 4 : 2;
     extern __shared__ __align__(16) uint8_t attn_lds[];
     __shared__ float msh[C::waves][32], lsh[C::waves][32];
-    __shared__ int bad_sh[C::waves];
+    __shared__ uint32_t bad_sh[C::waves];
     const int lane = static_cast<int>(threadIdx.x) & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
     const int rw = wave / KW, kw = wave % KW;
@@ -379,8 +332,8 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
 #pragma unroll
     for (int d = 0; d < ND; d++)
         unrolled<16>([&](auto ec) { chk = __builtin_fmaf(o[d][decltype(ec)::value], 0.0f, chk); });
-    uint64_t bad = __ballot(chk != 0.0f);  // NaN: some value is not finite
-    bool redo = bad != 0;                  // KW > 1: of any row group, so that every wave agrees
+    const uint64_t nan = __ballot(chk != 0.0f);  // NaN: some value is not finite
+    if (lane == 0) bad_sh[wave] = static_cast<uint32_t>(nan | (nan >> 32));
     // The KW waves of a row group: their states through LDS, merged in wave order; wave kw then finishes
     // the 32-dimension blocks kw, kw + KW, ...
     if constexpr (KW > 1) {
@@ -395,22 +348,25 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
             msh[wave][l32] = m;
             lsh[wave][l32] = l;
         }
-        if (lane == 0) bad_sh[wave] = static_cast<int>(bad | (bad >> 32));
-        __syncthreads();
-        redo = false;
+    }
+    __syncthreads();
+    uint32_t bad = 0, any_bad = 0;  // this row group's rows, and any group's
 #pragma unroll
-        for (int k = 0; k < C::waves; k++) redo |= bad_sh[k] != 0;
+    for (int k = 0; k < C::waves; k++) {
+        if (k / KW == rw) bad |= bad_sh[k];
+        any_bad |= bad_sh[k];
+    }
+    if constexpr (KW > 1) {
+        float* os = reinterpret_cast<float*>(attn_lds);
         float w[KW];
         m = kNoKey;
 #pragma unroll
         for (int k = 0; k < KW; k++) m = fmaxf(m, msh[rw * KW + k][l32]);
         l = 0.0f;
-        bad = 0;
 #pragma unroll
         for (int k = 0; k < KW; k++) {
             w[k] = __builtin_amdgcn_exp2f(msh[rw * KW + k][l32] - m);
             l = __builtin_fmaf(w[k], lsh[rw * KW + k][l32], l);
-            bad |= static_cast<uint32_t>(bad_sh[rw * KW + k]);
         }
 #pragma unroll
         for (int d = 0; d < ND; d++) {
@@ -424,7 +380,7 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
             });
         }
     }
-    const bool live = row0 + 32u * rw + l32 < n_rows;
+    const bool live = row0 + 32u * rw + l32 < n_rows && !((bad >> l32) & 1);
     const float inv = a.splits == 1 ? 1.0f / l : 1.0f;
     const int64_t th = t * a.n_head + head;
 #pragma unroll
@@ -457,19 +413,30 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
         pm[0] = l == 0.0f ? -INFINITY : m - kOffset;
         pm[1] = l;
     }
-    if (redo) {
-        if constexpr (KW > 1) __syncthreads();  // after the other waves' stores of these rows
-        if (kw != 0) return;
-        uint32_t rows = static_cast<uint32_t>(bad | (bad >> 32));
+    if (any_bad) {  // the same for the whole workgroup
+        typedef AttnItemLds<HD, C::waves, kRedoHeads> Lds;
+        static_assert(sizeof(Lds) <= C::lds, "LDS for the rows done again");
+        Lds& lds = *reinterpret_cast<Lds*>(attn_lds);
 #pragma unroll 1
-        while (rows) {
-            const int i = __builtin_ctz(rows);
-            rows &= rows - 1;
-            const uint32_t rr = row0 + 32u * rw + i;
-            if (rr >= n_rows) break;
-            const int64_t rt = rr / group;
-            const int rh = g * a.group + static_cast<int>(rr - static_cast<uint32_t>(rt) * group);
-            attend_row<TQ, HD>(a, rt, g, rh, k0, smaller(a.pos0 + rt + 1, k1), split);
+        for (int w = 0; w < RW; w++) {
+            uint32_t rows = 0;
+#pragma unroll
+            for (int k = 0; k < KW; k++) rows |= bad_sh[w * KW + k];
+#pragma unroll 1
+            while (rows) {
+                const int i = __builtin_ctz(rows);
+                const uint32_t rr = row0 + 32u * w + i;
+                if (rr >= n_rows) break;
+                const int64_t rt = rr / group;
+                const int rh = static_cast<int>(rr - static_cast<uint32_t>(rt) * group);
+                // The heads of this token that follow in the group of rows, too.
+                const uint32_t rest = ~(rows >> i);
+                const int run = min(rest ? __builtin_ctz(rest) : 32, min(kRedoHeads, a.group - rh));
+                rows &= ~(((1u << run) - 1) << i);
+                __syncthreads();  // the LDS before it
+                attend_item<TQ, HD, true, C::waves, kRedoHeads, false, true>(a, lds, rt, g, g * a.group + rh, run, split, k0,
+                                                                           smaller(a.pos0 + rt + 1, k1));
+            }
         }
     }
 }

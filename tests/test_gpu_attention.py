@@ -233,6 +233,12 @@ def test_attention_captured(dev, T, H, KV, hd, pos0, warm):
     (1, 8, 2, 128, 200, 100),      # one workgroup per head: three waves see only such keys
     (1, 8, 2, 96, 9000, 3000),     # whole splits
     (300, 8, 2, 96, 0, 70),        # no splits: the first 70 tokens see nothing else
+    (12, 8, 2, 128, 2000, 200),    # the matrix cores: some waves and splits see only such keys
+    (2, 8, 2, 128, 9000, 3000),    # whole splits
+    (40, 8, 2, 64, 900, 130),
+    (43, 6, 2, 128, 515, 150),     # rows done again: three heads of a token, across waves and row tiles
+    (129, 12, 12, 64, 0, 70),      # one head each
+    (70, 16, 1, 128, 400, 130),    # sixteen: items of four
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("low", [-float("inf"), float("nan")])
