@@ -29,8 +29,14 @@ struct AttnArgs {
     float* part;         // splits > 1: [T][n_head][splits][hd + 2] = (max, sum, accumulators)
 };
 
+constexpr float kLog2e = 1.44269504088896341f;
+// Base-2 exponents past which f32 no longer places a row's maximum well: within 2^20 its steps are 1/8.
+constexpr float kAttnFar = 1 << 20;
+
 // Partial results of a key split (splits > 1): the accumulators [T][n_head][splits][hd] at part, then
-// (max, sum) pairs [T][n_head][splits][2] after them.
+// (max, sum) pairs [T][n_head][splits][2] after them. The matrix-core path's maxima are base-2 exponents, but
+// those past kAttnFar are kept as the scores themselves, which are then exact against each other; such a
+// pair's sum has its sign bit set.
 __device__ __forceinline__ float* part_acc(const AttnArgs& a, int64_t th, int split) {
     return a.part + (th * a.splits + split) * a.hd;
 }

@@ -78,12 +78,39 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
         const float* pm = part_ml(a, th, min(s, S - 1));
         ms[k] = s < S ? pm[0] : -INFINITY;
         ls[k] = s < S ? pm[1] : 0.0f;
-        mx = fmaxf(mx, ms[k]);
+        // (LOG2: a maximum kept as a score counts as inf)
+        mx = fmaxf(mx, LOG2 && __builtin_signbitf(ls[k]) ? INFINITY : ms[k]);
     }
-    mx = wave_max_f32(mx);
-    if ((tid & 63) == 0) red[0][wave] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));  // above -inf: split 0 holds key 0
+    auto block_max = [&](float v) {
+        v = wave_max_f32(v);
+        if ((tid & 63) == 0) red[0][wave] = v;
+        __syncthreads();
+        return fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    };
+    mx = block_max(mx);  // above -inf: split 0 holds key 0
+    if (LOG2 && mx == INFINITY) {
+        // Scores among the maxima: all brought to one unit -- scores, if the largest is one (exponents are then too
+        // far below to matter), else exponents (and the scores are).
+        float ms_score = -INFINITY, ms_exp = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            float& m = __builtin_signbitf(ls[k]) ? ms_score : ms_exp;
+            m = fmaxf(m, ms[k]);
+        }
+        __syncthreads();  // red is read above
+        ms_score = block_max(ms_score);
+        __syncthreads();
+        ms_exp = block_max(ms_exp);
+        const bool scores = ms_score > ms_exp * (1.0f / kLog2e);
+        mx = scores ? 0.0f : ms_exp;
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const bool score = __builtin_signbitf(ls[k]);
+            if (scores) ms[k] = score ? (ms[k] - ms_score) * kLog2e : ms[k] - ms_score * kLog2e;
+            else if (score) ms[k] *= kLog2e;
+            ls[k] = fabsf(ls[k]);
+        }
+    }
     float sum = 0.0f;
 #pragma unroll
     for (int k = 0; k < kPer; k++) {

@@ -64,7 +64,7 @@ struct AttnItemLds {
 };
 
 // Query heads h0 .. h0 + nh - 1 (nh <= HB, all of kv head g) of token t over keys [k0, k1): into out, or as the
-// partial results of `split` where a.splits > 1 (LOG2: with the maximum as a base-2 exponent). Called by the
+// partial results of `split` where a.splits > 1 (LOG2: the matrix-core path's). Called by the
 // whole workgroup; lds is free for other use after the next barrier.
 template <typename TQ, int HDP, bool AL, int NW, int HB, bool PF, bool LOG2>
 __device__ __forceinline__ void attend_item(const AttnArgs& a, AttnItemLds<HDP, NW, HB>& lds, int64_t t, int g, int h0, int nh,
@@ -246,8 +246,11 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, AttnItemLds<HDP, 
                 if (d0 + e < hd) pa[d0 + e] = o[e];
             if (lane == 0) {
                 float* pm = part_ml(a, th, split);
-                pm[0] = LOG2 ? mx * 1.44269504088896341f : mx;
-                pm[1] = sum;
+                const float e2 = mx * kLog2e;
+                // (-FLT_MAX: no score above -inf)
+                const bool as_score = !LOG2 || (fabsf(e2) > kAttnFar && mx > -FLT_MAX);
+                pm[0] = as_score ? mx : e2;
+                pm[1] = LOG2 && as_score ? __builtin_copysignf(sum, -1.0f) : sum;
             }
         }
     }

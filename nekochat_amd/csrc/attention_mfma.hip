@@ -16,9 +16,10 @@
 // f32. The running maximum is kept as an integer exponent, in which rescaling and merging are exact,
 // and raised only when a score exceeds it by 8.
 // Rows whose result is not finite (an infinity or NaN among the inputs may have met a zero weight or
-// the other plane of a split) are done again by the workgroup as the vector path's items (attend_item). Where
-// that takes every row a call costs more than the vector path alone would (one infinite v, f16; 32 / 8 heads of
-// 128: 8192 tokens 24.1 ms and 22.3, 2048 tokens 2.65 and 1.59, 1 over 32768 keys 70 us and 53; 12 heads of
+// the other plane of a split), or whose scores pass 2^20 in log2 (from 2^24 the rounded maximum and the fma's
+// exact product part, by any power of two), are done again by the workgroup as the vector path's items
+// (attend_item). Where that takes every row a call costs more than the vector path alone would (one infinite v,
+// f16; 32 / 8 heads of 128: 8192 tokens 24.1 ms and 22.3, 2048 tokens 2.65 and 1.59, 1 over 32768 keys 70 us and 53; 12 heads of
 // 64, 1024 tokens, 570 and 215): a workgroup does its 128 rows one after the other and waits for each step's
 // loads. Loading ahead would take the registers of a second workgroup per CU from every call.
 //
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
         const TQ* qr = static_cast<const TQ*>(a.q) + t * a.qs + static_cast<int64_t>(head) * HD;
         // Position 0 has one key, of weight 1 whatever its score: a zero score makes that exact.
         const float sign = a.scale == 0.0f || a.pos0 + t == 0 ? 0.0f : a.scale < 0.0f ? -1.0f : 1.0f;
-        c = (a.scale == 0.0f ? 1.0f : fabsf(a.scale)) * 1.44269504088896341f;
+        c = (a.scale == 0.0f ? 1.0f : fabsf(a.scale)) * kLog2e;
         float x[NS][8];
 #pragma unroll
         for (int s = 0; s < NS; s++) {
@@ -336,8 +337,11 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
 #pragma unroll
     for (int d = 0; d < ND; d++)
         unrolled<16>([&](auto ec) { chk = __builtin_fmaf(o[d][decltype(ec)::value], 0.0f, chk); });
-    const uint64_t nan = __ballot(chk != 0.0f);  // NaN: some value is not finite
-    if (lane == 0) bad_sh[wave] = static_cast<uint32_t>(nan | (nan >> 32));
+    // Done again: rows with a value that is not finite (chk is NaN), and rows whose scores here lie too far out
+    // for the exponents (below kNoKey they leave every weight 0).
+    const bool far = fabsf(m) > kAttnFar && limit > k0 + 32 * KB_ * kw;
+    const uint64_t again = __ballot(chk != 0.0f || far);
+    if (lane == 0) bad_sh[wave] = static_cast<uint32_t>(again | (again >> 32));
     // The KW waves of a row group: their states through LDS, merged in wave order; wave kw then finishes
     // the 32-dimension blocks kw, kw + KW, ...
     if constexpr (KW > 1) {

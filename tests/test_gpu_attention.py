@@ -258,6 +258,31 @@ def test_attention_infinite_prefix(dev, T, H, KV, hd, pos0, n, dtype, low):
     assert (np.abs(got - want)[ok] <= bar * (1 + np.abs(want[ok]))).all()
 
 
+@pytest.mark.parametrize("T,H,KV,hd,pos0", [(1, 32, 8, 128, 5000), (24, 16, 8, 128, 600), (130, 8, 2, 64, 300)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("size", [-1e4, -1e8, -2e9, -1e12, -1e30, 1e8, 2e9, 1e12, 1e30])
+def test_attention_extreme_scores(dev, T, H, KV, hd, pos0, dtype, size):
+    """Scores of about 10 times `size` (f32 q of that size, or an f16 q under such a scale), apart by more than
+    any weight survives: only the keys of the largest weigh, all alike."""
+    _case(f"attention extreme scores T={T} H={H} KV={KV} hd={hd} pos0={pos0} {dtype} {size}")
+    _, kc, vc = _inputs(T, H, KV, hd, pos0, dev, seed=T + pos0)
+    level = torch.arange(pos0 + T, device=dev) % 7
+    kc[:] = (1.0 + level / 8.0)[:, None].half()
+    heads = (1.0 + torch.arange(H, device=dev) / 64.0).repeat_interleave(hd).repeat(T, 1)
+    heads = heads if size > 0 else -heads
+    if dtype == torch.float32:
+        out = ops.attention(heads * abs(size), kc, vc, H, KV, hd, pos0)
+    else:
+        out = ops.attention(heads.half(), kc, vc, H, KV, hd, pos0, scale=abs(size) / hd ** 0.5)
+    torch.cuda.synchronize()
+    v = vc.double().cpu()
+    for t in (0, T // 2, T - 1):
+        want = v[: pos0 + t + 1][(level[: pos0 + t + 1] == (0 if size < 0 else 6)).cpu()].mean(0)
+        want = torch.cat([want[(h // (H // KV)) * hd:(h // (H // KV) + 1) * hd] for h in range(H)])
+        bar = TOL if dtype == torch.float32 else 5e-4  # an f16 rounding: 2^-11
+        assert ((out[t].double().cpu() - want).abs() <= bar * (1 + want.abs())).all()
+
+
 def test_attention_argument_checks(dev):
     _case("attention argument checks")
     q, kc, vc = _inputs(2, 4, 2, 64, 5, dev, seed=5)
