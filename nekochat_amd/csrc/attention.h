@@ -34,9 +34,11 @@ constexpr float kLog2e = 1.44269504088896341f;
 constexpr float kAttnFar = 1 << 20;
 
 // Partial results of a key split (splits > 1): the accumulators [T][n_head][splits][hd] at part, then
-// (max, sum) pairs [T][n_head][splits][2] after them. The matrix-core path's maxima are base-2 exponents, but
-// those past kAttnFar are kept as the scores themselves, which are then exact against each other; such a
-// pair's sum has its sign bit set.
+// (max, sum) pairs [T][n_head][splits][2] after them. The matrix-core path's maxima are base-2 exponents,
+// halved; those past kAttnFar are kept as the scores themselves, which are then exact against each other.
+// kAttnScore tells them apart: exponents within 2^20 (and the weights' 2^15) halve to 2^19 + 8 at most,
+// scores past it are larger than 2^20 / log2(e) = 726817.
+constexpr float kAttnScore = 600000.0f;
 __device__ __forceinline__ float* part_acc(const AttnArgs& a, int64_t th, int split) {
     return a.part + (th * a.splits + split) * a.hd;
 }

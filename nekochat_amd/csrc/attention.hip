@@ -78,45 +78,26 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
         const float* pm = part_ml(a, th, min(s, S - 1));
         ms[k] = s < S ? pm[0] : -INFINITY;
         ls[k] = s < S ? pm[1] : 0.0f;
-        // (LOG2: a maximum kept as a score counts as inf)
-        mx = fmaxf(mx, LOG2 && __builtin_signbitf(ls[k]) ? INFINITY : ms[k]);
+        mx = fmaxf(mx, ms[k]);
     }
-    auto block_max = [&](float v) {
-        v = wave_max_f32(v);
-        if ((tid & 63) == 0) red[0][wave] = v;
-        __syncthreads();
-        return fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
-    };
-    mx = block_max(mx);  // above -inf: split 0 holds key 0
-    if (LOG2 && mx == INFINITY) {
-        // Scores among the maxima: all brought to one unit -- scores, if the largest is one (exponents are then too
-        // far below to matter), else exponents (and the scores are).
-        float ms_score = -INFINITY, ms_exp = -INFINITY;
+    mx = wave_max_f32(mx);
+    if ((tid & 63) == 0) red[0][wave] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));  // above -inf: split 0 holds key 0
+    if (LOG2 && fabsf(mx) > kAttnScore) {
+        // The largest is a score, and scores are taken from it as such. (Where an exponent is the largest, any
+        // scores lie so far below that their weights are 0, in whichever unit.)
 #pragma unroll
-        for (int k = 0; k < kPer; k++) {
-            float& m = __builtin_signbitf(ls[k]) ? ms_score : ms_exp;
-            m = fmaxf(m, ms[k]);
-        }
-        __syncthreads();  // red is read above
-        ms_score = block_max(ms_score);
-        __syncthreads();
-        ms_exp = block_max(ms_exp);
-        const bool scores = ms_score > ms_exp * (1.0f / kLog2e);
-        mx = scores ? 0.0f : ms_exp;
-#pragma unroll
-        for (int k = 0; k < kPer; k++) {
-            const bool score = __builtin_signbitf(ls[k]);
-            if (scores) ms[k] = score ? (ms[k] - ms_score) * kLog2e : ms[k] - ms_score * kLog2e;
-            else if (score) ms[k] *= kLog2e;
-            ls[k] = fabsf(ls[k]);
-        }
+        for (int k = 0; k < kPer; k++)
+            ms[k] = fabsf(ms[k]) > kAttnScore ? 0.5f * kLog2e * (ms[k] - mx) : ms[k] - 0.5f * kLog2e * mx;
+        mx = 0.0f;
     }
     float sum = 0.0f;
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
         const int s = tid + 256 * k;
-        // An empty split or none: exp(-inf) = 0.
-        const float ws = LOG2 ? __builtin_amdgcn_exp2f(ms[k] - mx) : expf(ms[k] - mx);
+        // An empty split or none: exp(-inf) = 0. (A NaN row ends here: -inf - -inf.)
+        const float ws = LOG2 ? __builtin_amdgcn_exp2f(__builtin_fmaf(2.0f, ms[k], -2.0f * mx)) : expf(ms[k] - mx);
         if (s < S) wsh[s] = ws;
         sum = __builtin_fmaf(ws, ls[k], sum);
     }

@@ -247,10 +247,8 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, AttnItemLds<HDP, 
             if (lane == 0) {
                 float* pm = part_ml(a, th, split);
                 const float e2 = mx * kLog2e;
-                // (-FLT_MAX: no score above -inf)
-                const bool as_score = !LOG2 || (fabsf(e2) > kAttnFar && mx > -FLT_MAX);
-                pm[0] = as_score ? mx : e2;
-                pm[1] = LOG2 && as_score ? __builtin_copysignf(sum, -1.0f) : sum;
+                pm[0] = !LOG2 || fabsf(e2) > kAttnFar ? mx : 0.5f * e2;
+                pm[1] = sum;
             }
         }
     }

@@ -357,14 +357,12 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
             lsh[wave][l32] = l;
         }
     }
-    __syncthreads();
-    uint32_t bad = 0, any_bad = 0;  // this row group's rows, and any group's
-#pragma unroll
-    for (int k = 0; k < C::waves; k++) {
-        if (k / KW == rw) bad |= bad_sh[k];
-        any_bad |= bad_sh[k];
-    }
+    // This row group's rows to do again.
+    uint32_t bad = static_cast<uint32_t>(again | (again >> 32));
     if constexpr (KW > 1) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < KW; k++) bad |= bad_sh[rw * KW + k];
         float* os = reinterpret_cast<float*>(attn_lds);
         float w[KW];
         m = kNoKey;
@@ -418,10 +416,14 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
     }
     if (a.splits > 1 && live && h == 0 && kw == 0) {
         float* pm = part_ml(a, th, split);
-        pm[0] = l == 0.0f ? -INFINITY : m - kOffset;
+        pm[0] = l == 0.0f ? -INFINITY : 0.5f * (m - kOffset);
         pm[1] = l;
     }
-    if (any_bad) {  // the same for the whole workgroup
+    if constexpr (KW == 1) __syncthreads();
+    uint32_t any_bad = 0;  // the same for the whole workgroup
+#pragma unroll
+    for (int k = 0; k < C::waves; k++) any_bad |= bad_sh[k];
+    if (any_bad) {
         typedef AttnItemLds<HD, C::waves, kRedoHeads> Lds;
         static_assert(sizeof(Lds) <= C::lds, "LDS for the rows done again");
         Lds& lds = *reinterpret_cast<Lds*>(attn_lds);
