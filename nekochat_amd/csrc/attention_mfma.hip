@@ -194,10 +194,10 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
 #pragma unroll
         for (int i = 0; i < C::loads; i++) {
             const int first = (wave * C::loads + i) * C::rpi;
-            // Opaque, so that the lane's offsets are computed per tile: kept, their registers spilled in the f32,
-            // 128-wide prompt kernel (seven reloads per tile; 8192 tokens 1077 us, 1022 without).
+            // Opaque in the f32, 128-wide prompt kernel, so that the lane's offsets are computed per tile: kept, their
+            // registers spilled (seven reloads per tile; 8192 tokens 1077 us, 1022 without).
             int row = lr;
-            asm volatile("" : "+v"(row));
+            if constexpr (kTwo && HD == 128 && KW == 1) asm volatile("" : "+v"(row));
             const uint32_t r = static_cast<uint32_t>(first + row);
             const uint32_t off = min(r, last) * row_bytes;
             // (address-space conversions: C casts, which reinterpret_cast does not allow)
