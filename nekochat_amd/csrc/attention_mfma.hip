@@ -11,17 +11,22 @@
 // which gives lane i of 16 column i of four rows. K and V reach LDS by global_load_lds, double
 // buffered, in chunk orders (k_slot, v_slot) that keep both kinds of read on distinct banks.
 //
-// Precision: f32 q rows are scaled by a power of two and split into two f16 (23 bits), probabilities
-// likewise (p 2^6 <= 2^14, two f16), K and V are f16 as stored; every product is exact and summed in
-// f32. The running maximum is kept as an integer exponent, in which rescaling and merging are exact,
-// and raised only when a score exceeds it by 8.
+// Precision: f32 q rows are scaled by a power of two and split into two f16 (24 bits of every element within
+// 2^-16 of the row's largest, 2^-39 of that below), K and V are f16 as stored, and products are exact and
+// summed in f32. Probabilities are split likewise, times 2^15: 24 bits above 2^-16 of the row's largest and
+// 2^-39 of it below, where f32 would keep 24 bits. The running maximum, an integer exponent in which rescaling
+// and merging are exact, is raised whenever a tile passes it, so that the scale is the largest f16 holds, and
+// the scale joins after the exponential, whose argument's rounding is thus that of a number near 0. Measured
+// as the sum of 8192 weights 22 nats below one dominant key, f32: off by 17% with a scale of 2^6 and a maximum
+// left alone by less than 8, by 1.4e-5 now; 8192 random keys 2.8e-7 (3.0e-7 then, 3.4e-7 with the scale in the
+// argument, 3.6e-7 on the vector path).
 // Rows whose result is not finite (an infinity or NaN among the inputs may have met a zero weight or
 // the other plane of a split), or whose scores pass 2^20 in log2 (from 2^24 the rounded maximum and the fma's
 // exact product part, by any power of two), are done again by the workgroup as the vector path's items
 // (attend_item). Where that takes every row a call costs more than the vector path alone would (one infinite v,
-// f16; 32 / 8 heads of 128: 8192 tokens 24.1 ms and 22.3, 2048 tokens 2.65 and 1.59, 1 over 32768 keys 70 us and 53; 12 heads of
-// 64, 1024 tokens, 570 and 215): a workgroup does its 128 rows one after the other and waits for each step's
-// loads. Loading ahead would take the registers of a second workgroup per CU from every call.
+// f16; 32 / 8 heads of 128: 8192 tokens 24.1 ms and 22.3, 2048 tokens 2.65 and 1.59, 1 over 32768 keys 70 us and
+// 53; 12 heads of 64, 1024 tokens, 570 and 215): a workgroup does its 128 rows one after the other and waits for
+// each step's loads. Loading ahead would take the registers of a second workgroup per CU from every call.
 //
 // What bounds it: the MFMAs -- the work counted twice in both products with f32 q, in one with f16 q -- with
 // the softmax's ~11 VALU operations per score beside them from the second wave of each SIMD. Measured
@@ -36,8 +41,8 @@
 namespace neko_hip {
 namespace {
 
-constexpr int kRaise = 8;    // the maximum is raised when a score exceeds it by more (in log2)
-constexpr int kOffset = 6;   // probabilities are held times 2^kOffset: <= 2^14, within f16
+constexpr int kOffset = 15;  // probabilities are split times 2^kOffset, the largest power that f16 holds
+constexpr float kScale = 1 << kOffset;
 constexpr double kMinWorkF16 = 70000, kMinWorkF32 = 112000, kMinPromptWork = 28000, kPromptRows = 100;  // see attn_mfma_takes
 constexpr int kRedoHeads = 4;     // query heads per item of the rows done again, at most
 constexpr float kNoKey = -1e30f;  // the running maximum before the first key
@@ -267,13 +272,12 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
             });
         const float top = half_swap_max(mx) * c;
         float corr = 1.0f;
-        if (__any(top > m + kRaise)) {
+        if (__any(top > m)) {
             const float mn = fmaxf(m, ceilf(top));
             corr = __builtin_amdgcn_exp2f(m - mn);
             m = mn;
         }
-        const float off = kOffset - m;
-        // p 2^kOffset, its sum, and its two planes by pairs.
+        // p, its sum, and its two planes.
         half8 ph[KB_][2], pl[KB_][2];
         float sum = 0.0f;  // of the tile, from zero: the row sum takes one rounding per tile
 #pragma unroll
@@ -285,13 +289,15 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
                     constexpr int e = decltype(ec)::value;
                     // The exponent, its parts joined by fmas towards the small value that it is for the
                     // keys that matter.
-                    float y = off;
+                    float y = -m;
 #pragma unroll
                     for (int n = NC - 1; n >= 0; n--) y = __builtin_fmaf(s[b][n][8 * i + e], c, y);
                     p[e] = __builtin_amdgcn_exp2f(y);
-                    const half_t hi = static_cast<half_t>(p[e]);
+                    float q = p[e] * kScale;
+                    asm("" : "+v"(q));  // opaque: folded into the conversion it is slower (8192 tokens, f16, 2%)
+                    const half_t hi = static_cast<half_t>(q);
                     ph[b][i][e] = hi;
-                    pl[b][i][e] = static_cast<half_t>(__builtin_fmaf(to_f32(hi), -1.0f, p[e]));
+                    pl[b][i][e] = static_cast<half_t>(__builtin_fmaf(p[e], kScale, -to_f32(hi)));
                 });
                 sum += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
             });
@@ -332,7 +338,7 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
         __syncthreads();                // and every wave's; this tile's reads are done
     }
 
-    l = half_swap_sum(l);
+    l = half_swap_sum(l) * kScale;  // in the accumulators' unit
     float chk = l * 0.0f;
 #pragma unroll
     for (int d = 0; d < ND; d++)

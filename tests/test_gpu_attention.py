@@ -283,6 +283,33 @@ def test_attention_extreme_scores(dev, T, H, KV, hd, pos0, dtype, size):
         assert ((out[t].double().cpu() - want).abs() <= bar * (1 + want.abs())).all()
 
 
+@pytest.mark.parametrize("gap", [14.0, 18.0, 21.0, 22.0, 26.0])
+@pytest.mark.parametrize("KV,keys,hd", [(2, 32768, 128), (2, 32768, 64), (520, 8192, 64), (260, 8192, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_attention_dominant_key(dev, KV, keys, hd, gap, dtype):
+    """One key `gap` nats above all others, its v zero and theirs of mean 1: the output is their weights' sum.
+    Every kv head holds the same, so that few (keys split) and many (not) share a reference in 64 bits. The
+    bar: the f32 bar, relative here, and a weight's rounding of 2^-39 of the largest for every key."""
+    _case(f"attention dominant key KV={KV} keys={keys} hd={hd} gap={gap} {dtype}")
+    g = torch.Generator().manual_seed(int(gap) + hd)
+    k, v = 0.25 * torch.randn((keys, hd), generator=g), 1.0 + 0.25 * torch.randn((keys, hd), generator=g)
+    q = 0.25 * torch.randn((1, hd), generator=g)
+    sink = keys // 3
+    k[:, 0] = 0.0
+    k[sink] = v[sink] = 0.0
+    k[sink, 0], q[0, 0] = 8.0, gap * hd ** 0.5 / 8.0
+    k, v, q = k.half(), v.half(), q.to(dtype)
+    s = (k.double() @ q[0].double()) / hd ** 0.5
+    want = torch.softmax(s, 0) @ v.double()
+    out = ops.attention(q.to(dev).repeat(1, KV), k.to(dev).repeat(1, KV), v.to(dev).repeat(1, KV), KV, KV, hd, keys - 1)
+    torch.cuda.synchronize()
+    err = (out.double().cpu().reshape(KV, hd) - want).abs()
+    if dtype == torch.float16:
+        err -= torch.from_numpy(np.spacing(np.abs(want.numpy()).astype(np.float16)).astype(np.float64)) / 2
+    print(f"worst error {err.max():.3e} of {want.abs().max():.3e}", flush=True)
+    assert (err <= TOL * want.abs() + keys * 2.0 ** -39).all()
+
+
 def test_attention_argument_checks(dev):
     _case("attention argument checks")
     q, kc, vc = _inputs(2, 4, 2, 64, 5, dev, seed=5)
