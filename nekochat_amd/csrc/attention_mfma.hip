@@ -83,12 +83,16 @@ struct MfmaTile {
     static constexpr int chunks = HD / 8;             // 16-byte chunks per row
     static constexpr int rpi = 64 / chunks;           // rows one wave's load instruction fills
     static constexpr int loads = keys / rpi / waves;  // load instructions per wave, tile and operand
+    // Workgroups per CU, by LDS (160 KB) and registers: f32 q of 128 dimensions with a row group's keys over
+    // several waves takes more than half a SIMD's. The kernel is compiled for as many, and the plan counts them.
+    template <typename TQ>
+    static constexpr int resident = 2 * (lds + 2048) <= 160 * 1024 && !(sizeof(TQ) == 4 && HD == 128 && KW > 1) ? 2 : 1;
     static_assert(KW == 1 || waves * 64 * (HD / 2) * 4 <= lds, "merge scratch");
     static_assert(keys % (rpi * waves) == 0, "whole load instructions");
 };
 
 template <typename TQ, int HD, int RW, int KW, int KB_>
-__global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kernel(AttnArgs a, int row_tiles, int vec_io) {
+__global__ __launch_bounds__(64 * RW * KW, (MfmaTile<HD, RW, KW, KB_>::template resident<TQ>)) void attn_mfma_kernel(AttnArgs a, int row_tiles, int vec_io) {
     typedef MfmaTile<HD, RW, KW, KB_> C;
     constexpr bool kTwo = sizeof(TQ) == 4;  // q in two f16 planes
     constexpr int NS = HD / 16, ND = HD / 32;
@@ -458,7 +462,7 @@ __global__ __launch_bounds__(64 * RW * KW, KW == 1 ? 2 : 1) void attn_mfma_kerne
 }
 
 template <typename TQ, int HD, int RW, int KW, int KB_>
-int launch(neko_hip_ctx* ctx, const AttnArgs& a, int row_tiles, bool vec_io) {
+int launch(neko_hip_ctx* ctx, const AttnArgs& a, MfmaTile<HD, RW, KW, KB_>, int row_tiles, bool vec_io) {
     typedef MfmaTile<HD, RW, KW, KB_> C;
     auto* kernel = &attn_mfma_kernel<TQ, HD, RW, KW, KB_>;
     static std::atomic<uint64_t> allowed{0};
@@ -469,13 +473,27 @@ int launch(neko_hip_ctx* ctx, const AttnArgs& a, int row_tiles, bool vec_io) {
     return NEKO_OK;
 }
 
+// The tiles of a call with rw row groups per workgroup: f(MfmaTile{}).
+template <int HD, typename F>
+auto with_tile(int rw, F f) {
+    switch (rw) {
+        case 1: return f(MfmaTile<HD, 1, 4, 1>{});
+        case 2: return f(MfmaTile<HD, 2, 2, 1>{});
+        default: return f(MfmaTile<HD, 4, 1, 2>{});
+    }
+}
+
 template <typename TQ, int HD>
 int launch_rows(neko_hip_ctx* ctx, const AttnArgs& a, int rw, int row_tiles, bool vec_io) {
-    switch (rw) {
-        case 1: return launch<TQ, HD, 1, 4, 1>(ctx, a, row_tiles, vec_io);
-        case 2: return launch<TQ, HD, 2, 2, 1>(ctx, a, row_tiles, vec_io);
-        default: return launch<TQ, HD, 4, 1, 2>(ctx, a, row_tiles, vec_io);
-    }
+    return with_tile<HD>(rw, [&](auto tile) { return launch<TQ>(ctx, a, tile, row_tiles, vec_io); });
+}
+
+int resident(int dtype, int hd, int rw) {
+    auto of = [&](auto tile) {
+        typedef decltype(tile) C;
+        return dtype == NEKO_DT_F16 ? C::template resident<half_t> : C::template resident<float>;
+    };
+    return hd == 64 ? with_tile<64>(rw, of) : with_tile<128>(rw, of);
 }
 
 }  // namespace
@@ -502,11 +520,11 @@ int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype) {
     const int64_t row_tiles = (rows + 32 * rw - 1) / (32 * rw);
     const int64_t tile_keys = rw == 1 ? 128 : 64;
     const int64_t tiles = (a.pos0 + a.T + tile_keys - 1) / tile_keys;
-    // Keys split until the launch holds the workgroups that fit at once (LDS: two per CU, one with 128-key
-    // tiles of 128-wide heads), each with at least two tiles (one where there is a single row group) --
-    // but not for four or fewer 64-key tiles (two of 128), which take no longer than the merge's
-    // launch, about 3.5 us.
-    const int64_t fit = static_cast<int64_t>(ctx->cu_count) * (rw == 1 && a.hd == 128 ? 1 : 2);
+    // Keys split until the launch holds the workgroups that fit at once (a second round would double the time:
+    // 12 tokens over 4000 keys, 32 / 8 heads of 128, f32, 16.4 us at one per CU and 25.6 split for two), each
+    // with at least two tiles (one where there is a single row group) -- but not for four or fewer 64-key tiles
+    // (two of 128), which take no longer than the merge's launch, about 3.5 us.
+    const int64_t fit = static_cast<int64_t>(ctx->cu_count) * resident(dtype, a.hd, rw);
     const int64_t wgs = row_tiles * a.n_kv;
     const int64_t most = tiles * tile_keys <= 256 ? 1 : rw == 4 ? tiles / 2 : tiles;
     int64_t splits = std::max<int64_t>(1, std::min<int64_t>({fit / wgs, most, kAttnMaxSplits}));
