@@ -70,8 +70,15 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 
 // Combines the splits of a.part into a.out (log2: the maxima are base-2 exponents).
 int attn_merge(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, int dtype, bool log2);
-// The matrix-core path (attention_mfma.hip): whether it takes this call, and its launches, where it does.
-bool attn_mfma_takes(const AttnArgs& a, int dtype);
-int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype);
+// The matrix-core path (attention_mfma.hip): whether it can take a call, how it would, and its launches.
+struct AttnMfmaPlan {
+    int row_groups;     // of 32 rows, per workgroup
+    int64_t row_tiles;  // of as many rows, per kv head
+    int64_t splits;     // of the keys
+    double us;          // estimated time, kv_us being that of reading K and V once (attention.hip: how measured)
+};
+bool attn_mfma_can(const AttnArgs& a);
+AttnMfmaPlan attn_mfma_plan(const neko_hip_ctx* ctx, const AttnArgs& a, int dtype, double kv_us);
+int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype, const AttnMfmaPlan& plan);
 
 }  // namespace neko_hip

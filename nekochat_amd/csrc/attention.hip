@@ -3,8 +3,8 @@
 // for token t at position pos0 + t and query head h, out = sum_j softmax_j(scale * q_h . k_j) v_j over
 // cache rows j <= pos0 + t, k_j / v_j being kv head h / (n_head / n_kv) of those rows.
 //
-// Calls with enough work take the matrix cores where the head size is 64 or 128 (attention_mfma.hip); what
-// follows is the vector path for the rest, whose work items attention_item.h computes.
+// Calls with heads of 64 or 128 take the matrix cores (attention_mfma.hip) where that is estimated to be faster;
+// what follows is the vector path for the rest, whose work items attention_item.h computes.
 //
 // A workgroup of four waves per work item (token, kv head, block of up to four of the query heads that
 // share it, split of the keys), the item's steps of keys dealt round robin to its waves. Lane = (key
@@ -167,6 +167,23 @@ int launch_typed(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, bool ve
     return launch_hdp<TQ, 256>(ctx, what, a, vec, items, one_head, wide);
 }
 
+// Estimated time of a call on the vector path: rounds of the workgroups that fit, each with a start and its
+// waves' steps (of the average row; an item of one query head hides its first in the start), or the reads of
+// K and V by every token and head block, and the merge.
+double vector_us(const neko_hip_ctx* ctx, const AttnArgs& a, bool one_head, bool wide, int64_t items, int64_t steps,
+                 double kv_us) {
+    const int64_t waves = wide ? kAttnWideWaves : kAttnWaves;
+    const int64_t per = ((steps + a.splits - 1) / a.splits + waves - 1) / waves;
+    const int fit = wide ? 2 : one_head ? 4 : per > 1 ? 2 : 3;  // workgroups per CU, by registers
+    const double rounds = std::max(1.0, static_cast<double>(items) / (static_cast<double>(ctx->cu_count) * fit));
+    const double rows = static_cast<double>(a.pos0) + 0.5 * static_cast<double>(a.T);
+    const double seen = rows / static_cast<double>(a.pos0 + a.T);
+    const double step = one_head ? 6.0 * static_cast<double>(per - 1)
+                                 : 1.6 * static_cast<double>(per) * std::min(a.group, kAttnHeads);
+    return 1.0 + std::max(rounds * (5.0 + seen * step), static_cast<double>(a.T * a.hblocks) * seen * kv_us) +
+           (a.splits > 1 ? 2.5 + 0.004 * static_cast<double>(a.T * a.n_head) * a.splits : 0.0);
+}
+
 }  // namespace
 
 int attn_merge(neko_hip_ctx* ctx, const char* what, const AttnArgs& a, int dtype, bool log2) {
@@ -227,8 +244,6 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
     a.hd = hd;
     a.scale = scale;
     NEKO_REQUIRE(ctx, T * n_head <= 0x7fffffff, "%s: grid too large", what);
-    // Before the vector path's plan, whose workspace these calls do not use.
-    if (attn_mfma_takes(a, dtype)) return attn_mfma(ctx, what, a, dtype);
     // One query head per item where the K and V rows are few (their re-reads by the group's heads stay
     // in L2) and the launch would otherwise be short of waves; else up to four heads share each load.
     const int64_t kv_bytes = (pos0 + T) * static_cast<int64_t>(n_kv) * hd * 4;
@@ -257,6 +272,18 @@ extern "C" int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_st
     a.split_keys = (steps + splits - 1) / splits * step;
     a.splits = static_cast<int>((keys + a.split_keys - 1) / a.split_keys);
     const int64_t items = base * a.splits;
+    // The matrix cores where their estimated time is the shorter. Both estimates were fitted to the same calls,
+    // each timed on both paths (1624 calls: 1 to 600 tokens, 16 shapes of heads, 4 thousand to 3 million pairs
+    // of a query head and a key, f16 and f32; rms 9% there and 15% here; K and V past the caches are read at 5.2
+    // TB/s). Over 400 calls of other sizes the choice costs 0.5% over the better path on average and is never more
+    // than 15% behind the vector path. A line drawn at a number of pairs cost 3.1%, and was behind by up to
+    // 2.1 times: 35 tokens over 155 keys, 6 / 2 heads of 128, f32, 6.3 us here and 13.3 there, while 57 tokens from
+    // 0, 32 / 32 heads, f16, take 16.3 here and 7.0 there. Asked before either path wants a workspace.
+    if (attn_mfma_can(a)) {
+        const double kv_us = kv_bytes > kAttnOneHeadBytes ? static_cast<double>(kv_bytes) / 5.2e6 : 0.0;
+        const AttnMfmaPlan plan = attn_mfma_plan(ctx, a, dtype, kv_us);
+        if (plan.us < vector_us(ctx, a, one_head, wide, items, steps, kv_us)) return attn_mfma(ctx, what, a, dtype, plan);
+    }
     NEKO_REQUIRE(ctx, items <= 0x7fffffff, "%s: grid too large", what);
     if (a.splits > 1) {
         void* ws = nullptr;

@@ -43,7 +43,6 @@ namespace {
 
 constexpr int kOffset = 15;  // probabilities are split times 2^kOffset, the largest power that f16 holds
 constexpr float kScale = 1 << kOffset;
-constexpr double kMinWorkF16 = 70000, kMinWorkF32 = 112000, kMinPromptWork = 28000, kPromptRows = 100;  // see attn_mfma_takes
 constexpr int kRedoHeads = 4;     // query heads per item of the rows done again, at most
 constexpr float kNoKey = -1e30f;  // the running maximum before the first key
 
@@ -114,7 +113,7 @@ __global__ __launch_bounds__(64 * RW * KW, (MfmaTile<HD, RW, KW, KB_>::template 
     const int split = static_cast<int>(item % static_cast<uint32_t>(a.splits));
     const int tile = row_tiles - 1 - static_cast<int>(item / static_cast<uint32_t>(a.splits));
     const uint32_t group = static_cast<uint32_t>(a.group);
-    const uint32_t n_rows = static_cast<uint32_t>(a.T) * group;  // below 2^31 (attn_mfma_takes)
+    const uint32_t n_rows = static_cast<uint32_t>(a.T) * group;  // below 2^31 (attn_mfma_can)
     const uint32_t row0 = static_cast<uint32_t>(tile) * C::rows;
 
     // The keys this workgroup sees, cut into a.splits runs of whole tiles.
@@ -190,7 +189,7 @@ __global__ __launch_bounds__(64 * RW * KW, (MfmaTile<HD, RW, KW, KB_>::template 
     // slot); the lane reads the chunk that belongs in its slot. Row offsets in 32 bits past a uniform
     // base; rows past the caches' end repeat the last.
     const int64_t cache_rows = a.pos0 + a.T;
-    const uint32_t row_bytes = static_cast<uint32_t>(a.kvw) * 2;  // below 2^21 (attn_mfma_takes)
+    const uint32_t row_bytes = static_cast<uint32_t>(a.kvw) * 2;  // below 2^21 (attn_mfma_can)
     const int lr = lane / C::chunks, ls = lane % C::chunks;
     const char* kbase = reinterpret_cast<const char*>(a.kc + static_cast<int64_t>(g) * HD);
     const char* vbase = reinterpret_cast<const char*>(a.vc + static_cast<int64_t>(g) * HD);
@@ -498,36 +497,40 @@ int resident(int dtype, int hd, int rw) {
 
 }  // namespace
 
-bool attn_mfma_takes(const AttnArgs& a, int dtype) {
+bool attn_mfma_can(const AttnArgs& a) {
     // 32-bit row numbers and offsets within a tile; whole 16-byte chunks.
-    if ((a.hd != 64 && a.hd != 128) || !aligned(a.kc, 16) || !aligned(a.vc, 16) || a.kvw > (1 << 20) ||
-        a.T * a.group >= (int64_t{1} << 31) - 256)
-        return false;
-    // From kMinWorkF16 / F32 query-head x key pairs of 128 dimensions; below, the vector path's shorter start wins:
-    // with 32 / 8 heads of 128, f16, 4 tokens over 504 keys (64 k pairs) take 11.0 us there and 11.6 here, 2
-    // over 1502 (96 k) 12.9 and 11.7, 1 over 4001 (128 k) 13.5 and 11.0, 8 over 508 (130 k) 12.9 and
-    // 10.4; f32, 12 tokens of 16 / 8 heads over 512 keys (97 k) 12.2 and 14.2, 1 of 32 / 8 over 4001 (128 k)
-    // 13.5 and 11.5. Prompts, whose rows fill the columns of several waves, from kMinPromptWork: 100 tokens
-    // from 0, 12 heads of 64 (30 k) 11.5 and 7.0.
-    const double rows = static_cast<double>(a.T) * a.group;
-    const double work = rows * a.n_kv * static_cast<double>(a.pos0 + (a.T + 1) / 2) / (128 / a.hd);
-    return work >= (rows >= kPromptRows ? kMinPromptWork : dtype == NEKO_DT_F16 ? kMinWorkF16 : kMinWorkF32);
+    return (a.hd == 64 || a.hd == 128) && aligned(a.kc, 16) && aligned(a.vc, 16) && a.kvw <= (1 << 20) &&
+           a.T * a.group < (int64_t{1} << 31) - 256;
 }
 
-int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype) {
+AttnMfmaPlan attn_mfma_plan(const neko_hip_ctx* ctx, const AttnArgs& a, int dtype, double kv_us) {
+    AttnMfmaPlan p;
     const int64_t rows = a.T * a.group;
-    const int rw = rows <= 32 ? 1 : rows <= 64 ? 2 : 4;
-    const int64_t row_tiles = (rows + 32 * rw - 1) / (32 * rw);
-    const int64_t tile_keys = rw == 1 ? 128 : 64;
+    p.row_groups = rows <= 32 ? 1 : rows <= 64 ? 2 : 4;
+    p.row_tiles = (rows + 32 * p.row_groups - 1) / (32 * p.row_groups);
+    const int64_t tile_keys = p.row_groups == 1 ? 128 : 64;
     const int64_t tiles = (a.pos0 + a.T + tile_keys - 1) / tile_keys;
     // Keys split until the launch holds the workgroups that fit at once (a second round would double the time:
     // 12 tokens over 4000 keys, 32 / 8 heads of 128, f32, 16.4 us at one per CU and 25.6 split for two), each
     // with at least two tiles (one where there is a single row group) -- but not for four or fewer 64-key tiles
     // (two of 128), which take no longer than the merge's launch, about 3.5 us.
-    const int64_t fit = static_cast<int64_t>(ctx->cu_count) * resident(dtype, a.hd, rw);
-    const int64_t wgs = row_tiles * a.n_kv;
-    const int64_t most = tiles * tile_keys <= 256 ? 1 : rw == 4 ? tiles / 2 : tiles;
-    int64_t splits = std::max<int64_t>(1, std::min<int64_t>({fit / wgs, most, kAttnMaxSplits}));
+    const int64_t fit = static_cast<int64_t>(ctx->cu_count) * resident(dtype, a.hd, p.row_groups);
+    const int64_t wgs = p.row_tiles * a.n_kv;
+    const int64_t most = tiles * tile_keys <= 256 ? 1 : p.row_groups == 4 ? tiles / 2 : tiles;
+    p.splits = std::max<int64_t>(1, std::min<int64_t>({fit / wgs, most, kAttnMaxSplits}));
+    // The start of a launch, a tile of 1, 2 or 4 row groups, by head size and type; rounds of workgroups; the merge.
+    static constexpr double kStart[2][2] = {{3.3, 3.8}, {5.1, 6.4}};
+    static constexpr double kTile[2][2][3] = {{{1.7, 1.0, 1.5}, {2.2, 1.5, 1.8}}, {{1.6, 1.4, 2.2}, {1.9, 2.0, 2.5}}};
+    const int wide = a.hd == 128, two = dtype == NEKO_DT_F32;
+    const double rounds = std::max(1.0, static_cast<double>(wgs * p.splits) / static_cast<double>(fit));
+    const double tile_us = rounds * static_cast<double>((tiles + p.splits - 1) / p.splits) * kTile[wide][two][p.row_groups / 2];
+    p.us = kStart[wide][two] + std::max(tile_us, kv_us) +
+           (p.splits > 1 ? 3.3 + 0.0003 * static_cast<double>(a.T * a.n_head * p.splits) : 0.0);
+    return p;
+}
+
+int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype, const AttnMfmaPlan& plan) {
+    int64_t splits = plan.splits;
     const int64_t split_bytes = a.T * a.n_head * (a.hd + 2) * static_cast<int64_t>(sizeof(float));
     // Under capture the workspace cannot grow: as many splits as it holds.
     if (splits > 1 && static_cast<size_t>(splits * split_bytes) > ctx->workspace_bytes[0]) {
@@ -542,10 +545,10 @@ int attn_mfma(neko_hip_ctx* ctx, const char* what, AttnArgs& a, int dtype) {
         if (int rc = workspace(ctx, static_cast<size_t>(splits * split_bytes), &ws)) return rc;
         a.part = static_cast<float*>(ws);
     }
-    NEKO_REQUIRE(ctx, wgs * splits <= 0x7fffffff, "%s: grid too large", what);
+    NEKO_REQUIRE(ctx, plan.row_tiles * a.n_kv * splits <= 0x7fffffff, "%s: grid too large", what);
     const size_t esz = dtype_size(dtype);
     const bool vec_io = aligned(a.q, 16) && aligned(a.out, 16) && a.qs * esz % 16 == 0 && a.os * esz % 16 == 0;
-    const int rt = static_cast<int>(row_tiles);
+    const int rw = plan.row_groups, rt = static_cast<int>(plan.row_tiles);
     int rc;
     if (dtype == NEKO_DT_F16) rc = a.hd == 64 ? launch_rows<half_t, 64>(ctx, a, rw, rt, vec_io) : launch_rows<half_t, 128>(ctx, a, rw, rt, vec_io);
     else rc = a.hd == 64 ? launch_rows<float, 64>(ctx, a, rw, rt, vec_io) : launch_rows<float, 128>(ctx, a, rw, rt, vec_io);

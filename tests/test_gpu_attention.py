@@ -131,15 +131,19 @@ def test_attention_scale_and_single_key(dev):
 # The matrix-core path (rows = tokens x query heads per kv head, 32 to a wave): one, two or four row groups
 # per workgroup and key tiles of 128 or 64, at their edges, split over the keys and not; then short rows.
 @pytest.mark.parametrize("T,H,KV,hd,pos0", [
-    (8, 128, 32, 128, 119),  # 32 rows, 127 keys: one row group, the key tile short of one
+    (8, 256, 64, 128, 119),  # 32 rows, 127 keys: one row group, the key tile short of one
+    (8, 128, 32, 128, 119),  # the same of half the heads: the vector path
     (8, 256, 64, 64, 121),   # 129 keys: one past a tile
     (16, 128, 32, 128, 48),  # 64 rows, 64 keys: two row groups
-    (17, 64, 16, 128, 100),  # 68 rows: four row groups, the third with 4 rows, the last empty
+    (17, 256, 64, 128, 100),  # 68 rows: four row groups, the third with 4 rows, the last empty
+    (17, 64, 16, 128, 100),  # a quarter of the heads: the vector path
     (32, 64, 16, 64, 33),    # 128 rows, 65 keys
     (33, 16, 4, 128, 640),   # 132 rows: a second row tile of 4 rows, keys split
     (43, 6, 2, 128, 515),    # three heads per kv head: tokens straddle waves and row tiles
     (129, 12, 12, 64, 0),    # one head per kv head
     (300, 16, 1, 128, 1),    # sixteen heads per kv head, splits empty for the first rows
+    (32, 8, 1, 128, 203),    # 256 rows of one kv head: the vector path
+    (50, 32, 32, 128, 0),    # as much work in 1600 items: the matrix cores
     (1, 8, 2, 128, 128),     # below: a head's whole row by eight waves; 129 keys, five waves with a step
     (2, 8, 2, 128, 254),     # 256 keys: every wave's step full
     (1, 8, 2, 128, 256),     # 257 keys: split again
@@ -258,7 +262,7 @@ def test_attention_infinite_prefix(dev, T, H, KV, hd, pos0, n, dtype, low):
     assert (np.abs(got - want)[ok] <= bar * (1 + np.abs(want[ok]))).all()
 
 
-@pytest.mark.parametrize("T,H,KV,hd,pos0", [(1, 32, 8, 128, 5000), (24, 16, 8, 128, 600), (130, 8, 2, 64, 300)])
+@pytest.mark.parametrize("T,H,KV,hd,pos0", [(1, 32, 8, 128, 5000), (24, 16, 8, 128, 600), (130, 16, 4, 64, 300)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("size", [-1e4, -1e8, -2e9, -1e12, -1e30, 1e8, 2e9, 1e12, 1e30])
 def test_attention_extreme_scores(dev, T, H, KV, hd, pos0, dtype, size):
@@ -284,13 +288,14 @@ def test_attention_extreme_scores(dev, T, H, KV, hd, pos0, dtype, size):
 
 
 @pytest.mark.parametrize("gap", [14.0, 18.0, 21.0, 22.0, 26.0])
-@pytest.mark.parametrize("KV,keys,hd", [(2, 32768, 128), (2, 32768, 64), (520, 8192, 64), (260, 8192, 128)])
+@pytest.mark.parametrize("H,KV,keys,hd", [(32, 8, 32768, 128), (16, 4, 32768, 64), (520, 520, 8192, 64),
+                                           (260, 260, 8192, 128)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
-def test_attention_dominant_key(dev, KV, keys, hd, gap, dtype):
+def test_attention_dominant_key(dev, H, KV, keys, hd, gap, dtype):
     """One key `gap` nats above all others, its v zero and theirs of mean 1: the output is their weights' sum.
     Every kv head holds the same, so that few (keys split) and many (not) share a reference in 64 bits. The
     bar: the f32 bar, relative here, and a weight's rounding of 2^-39 of the largest for every key."""
-    _case(f"attention dominant key KV={KV} keys={keys} hd={hd} gap={gap} {dtype}")
+    _case(f"attention dominant key H={H} KV={KV} keys={keys} hd={hd} gap={gap} {dtype}")
     g = torch.Generator().manual_seed(int(gap) + hd)
     k, v = 0.25 * torch.randn((keys, hd), generator=g), 1.0 + 0.25 * torch.randn((keys, hd), generator=g)
     q = 0.25 * torch.randn((1, hd), generator=g)
@@ -301,9 +306,9 @@ def test_attention_dominant_key(dev, KV, keys, hd, gap, dtype):
     k, v, q = k.half(), v.half(), q.to(dtype)
     s = (k.double() @ q[0].double()) / hd ** 0.5
     want = torch.softmax(s, 0) @ v.double()
-    out = ops.attention(q.to(dev).repeat(1, KV), k.to(dev).repeat(1, KV), v.to(dev).repeat(1, KV), KV, KV, hd, keys - 1)
+    out = ops.attention(q.to(dev).repeat(1, H), k.to(dev).repeat(1, KV), v.to(dev).repeat(1, KV), H, KV, hd, keys - 1)
     torch.cuda.synchronize()
-    err = (out.double().cpu().reshape(KV, hd) - want).abs()
+    err = (out.double().cpu().reshape(H, hd) - want).abs()
     if dtype == torch.float16:
         err -= torch.from_numpy(np.spacing(np.abs(want.numpy()).astype(np.float16)).astype(np.float64)) / 2
     print(f"worst error {err.max():.3e} of {want.abs().max():.3e}", flush=True)
