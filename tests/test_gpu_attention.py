@@ -7,9 +7,10 @@ in different orders -- so the bar is a tolerance, written below: |gpu - oracle| 
 with TOL = 2e-6 for f32 outputs (the reference's own self-test allows 2e-3), and f16 outputs within
 half an f16 ulp of the oracle's f32 result plus that bar. Shapes: the reference self-test case, the Qwen3-4B
 decode (one token over 4096 and 40000 cached positions: the keys split over many workgroups and
-merged; one kv head over 100000 positions: 391 splits) and a 256-token prefill, GPT-2 heads, head
-sizes 6 / 96 / 256 (the per-half and masked loads), groups of 3 and 8 query heads per kv head, work
-items of one and of four query heads, strided q / out rows, f16 activations, and the argument checks.
+merged) and a 256-token prefill, GPT-2 heads, head sizes 6 / 40 / 96 / 256 (the per-half and masked
+loads), groups of 3, 8 and 16 query heads per kv head, strided and unaligned q / out rows, f16
+activations, infinities, extreme scores, graph capture, and the argument checks. Heads of 64 and 128 run
+on the matrix cores where that is estimated to be faster, the rest on the vector path.
 """
 import numpy as np
 import pytest
@@ -54,9 +55,9 @@ def _check_f32(got, want, what):
 
 @pytest.mark.parametrize("T,H,KV,hd,pos0", [
     (3, 4, 2, 64, 1030),    # the reference self-test case (compute.cpp:262-283)
-    (1, 32, 8, 128, 4095),  # Qwen3-4B decode, 4096 cached positions: keys split over waves
+    (1, 32, 8, 128, 4095),  # Qwen3-4B decode, 4096 cached positions: 32 key splits
     (4, 32, 8, 128, 2000),  # four-sequence decode step
-    (256, 32, 8, 128, 0),   # Qwen3-4B prefill of 256 tokens: one item per (token, kv head)
+    (256, 32, 8, 128, 0),   # Qwen3-4B prefill of 256 tokens: eight row tiles per kv head
     (64, 12, 12, 64, 0),    # GPT-2 small: one query head per kv head
     (8, 8, 2, 256, 100),    # head size 256, one query head per work item
     (512, 8, 2, 256, 0),    # head size 256, four query heads per work item
@@ -64,10 +65,10 @@ def _check_f32(got, want, what):
     (3, 4, 2, 6, 9),        # head size 6: per-half loads, one query head per work item
     (512, 4, 2, 6, 0),      # head size 6, two query heads per work item
     (7, 12, 4, 64, 200),    # three query heads per kv head
-    (2, 16, 2, 128, 3000),  # eight query heads per kv head, one per work item
-    (1, 16, 2, 128, 40000),  # eight query heads per kv head: two blocks of four (41 MB of K and V)
-    (1, 32, 8, 128, 40000),  # long context: 126 splits merged
-    (1, 4, 1, 128, 100000),  # one kv head: 391 splits (the merge's threads each take several)
+    (2, 16, 2, 128, 3000),  # eight query heads per kv head
+    (1, 16, 2, 128, 40000),  # 128 key splits
+    (1, 32, 8, 128, 40000),  # long context: 32, of ten tiles
+    (1, 4, 1, 128, 100000),  # one kv head: 256
 ])
 def test_attention_f32(dev, T, H, KV, hd, pos0):
     _case(f"attention f32 T={T} H={H} KV={KV} hd={hd} pos0={pos0}")
@@ -313,6 +314,61 @@ def test_attention_dominant_key(dev, H, KV, keys, hd, gap, dtype):
         err -= torch.from_numpy(np.spacing(np.abs(want.numpy()).astype(np.float16)).astype(np.float64)) / 2
     print(f"worst error {err.max():.3e} of {want.abs().max():.3e}", flush=True)
     assert (err <= TOL * want.abs() + keys * 2.0 ** -39).all()
+
+
+@pytest.mark.parametrize("T,H,KV,hd,pos0", [
+    (9, 32, 8, 128, 700), (33, 16, 4, 128, 640), (130, 12, 12, 64, 20), (40, 12, 4, 64, 1500),
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("off,pad", [(0, 40), (1, 0), (0, 1), (1, 7)])
+def test_attention_mfma_layouts(dev, T, H, KV, hd, pos0, dtype, off, pad):
+    """The matrix-core path over q and out rows that are padded, off 16-byte alignment by one element, or of an odd
+    stride (element loads and stores); nothing beside the out rows is written."""
+    _case(f"attention layouts T={T} H={H} KV={KV} hd={hd} pos0={pos0} {dtype} off={off} pad={pad}")
+    q, kc, vc = _inputs(T, H, KV, hd, pos0, dev, seed=T + pos0)
+    W = H * hd
+    qfull = torch.full((off + T * (W + pad),), float("nan"), dtype=dtype, device=dev)
+    qs = qfull[off:].view(T, W + pad)[:, :W]
+    qs.copy_(q)
+    ofull = torch.full((off + T * (W + pad) + 8,), 7.0, dtype=dtype, device=dev)
+    o = ofull[off:-8].view(T, W + pad)
+    ops.attention(qs, kc, vc, H, KV, hd, pos0, out=o[:, :W])
+    torch.cuda.synchronize()
+    want = _oracle(qs.contiguous(), kc, vc, H, KV, hd, pos0)
+    half_ulp = 0 if dtype == torch.float32 else np.spacing(np.abs(want).astype(np.float16)).astype(np.float32) / 2
+    excess = np.abs(o[:, :W].float().cpu().numpy() - want) - half_ulp - TOL * (1.0 + np.abs(want))
+    assert (excess <= 0).all()
+    assert bool((o[:, W:] == 7.0).all()) and bool((ofull[:off] == 7.0).all()) and bool((ofull[-8:] == 7.0).all())
+
+
+@pytest.mark.parametrize("T,H,KV,hd,pos0", [(1, 32, 8, 128, 5000), (130, 12, 12, 64, 20)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_attention_mfma_zero_scale(dev, T, H, KV, hd, pos0, dtype):
+    """A zero scale on the matrix cores: the mean of the v rows, splits and prompts."""
+    _case(f"attention zero scale T={T} H={H} KV={KV} hd={hd} pos0={pos0} {dtype}")
+    q, kc, vc = _inputs(T, H, KV, hd, pos0, dev, seed=T)
+    out = ops.attention(q.to(dtype), kc, vc, H, KV, hd, pos0, scale=0.0)
+    torch.cuda.synchronize()
+    mean = vc.double().cumsum(0)[pos0:] / torch.arange(pos0 + 1, pos0 + T + 1, device=dev)[:, None]
+    want = mean.reshape(T, KV, 1, hd).expand(T, KV, H // KV, hd).reshape(T, H * hd)
+    bar = TOL if dtype == torch.float32 else 5e-4  # an f16 rounding: 2^-11
+    assert bool(((out.double() - want).abs() <= bar * (1 + want.abs())).all())
+
+
+@pytest.mark.parametrize("H,KV,hd,pos0", [
+    (1, 1, 96, 40000),    # 313 splits, each item one query head
+    (2, 1, 256, 30000),   # 469
+    (4, 1, 96, 100000),   # 782 splits of items of four query heads (38 MB of K and V)
+    (16, 2, 256, 40000),  # two blocks of four
+])
+def test_attention_vector_splits(dev, H, KV, hd, pos0):
+    """Head sizes of the vector path at long decode: splits past 256, which the merge's threads take several of,
+    and items of four query heads with split keys."""
+    _case(f"attention vector splits H={H} KV={KV} hd={hd} pos0={pos0}")
+    q, kc, vc = _inputs(1, H, KV, hd, pos0, dev, seed=hd + pos0)
+    out = ops.attention(q, kc, vc, H, KV, hd, pos0)
+    torch.cuda.synchronize()
+    _check_f32(out, _oracle(q, kc, vc, H, KV, hd, pos0), f"attention H={H} KV={KV} hd={hd} pos0={pos0}")
 
 
 def test_attention_argument_checks(dev):
