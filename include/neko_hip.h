@@ -146,11 +146,14 @@ int neko_hip_store_kv(neko_hip_ctx* ctx, const void* qkv, int64_t row_stride, in
  * rows of n_kv*hd halves, holding positions 0 .. pos0 + T - 1). n_head a multiple of n_kv; hd even,
  * 2..256; the reference's scale is 1/sqrt(hd); caches 4-byte aligned. out may not overlap q or the
  * caches. f32 sums in another order than the reference's CPU loop (whose order its own shader does not
- * follow either): within 1e-6 relative of it at the tested shapes.
+ * follow either), and calls with heads of 64 or 128 that are faster so run on the matrix cores, f32 q and the
+ * weights as two f16 each (24 bits, weights to 2^-39 of the row's largest). Tested to |out - cpu| <= 2e-6 (1 + |cpu|)
+ * for f32, half an f16 ulp more for f16. Infinities, NaN and scores of any finite size come out as the CPU
+ * loop's, at a few times the cost where they touch a row on the matrix cores.
  * Calls that split their keys over workgroups keep partial results in the context's workspace (see
- * neko_hip_matmul below). While the stream is under graph capture it cannot grow: the matrix-core calls (heads
- * of 64 or 128, larger calls) then take as many splits as it holds, down to one; the others fail with
- * NEKO_ERR_INVALID. One uncaptured call of the same shape first gives both what they need. */
+ * neko_hip_matmul below). While the stream is under graph capture it cannot grow: the matrix-core calls then
+ * take as many splits as it holds, down to one; the others fail with NEKO_ERR_INVALID. One uncaptured call of
+ * the same shape first gives both what they need. */
 int neko_hip_attention(neko_hip_ctx* ctx, const void* q, int64_t q_stride, const uint16_t* k_cache, const uint16_t* v_cache,
                        void* out, int64_t out_stride, int64_t T, int n_head, int n_kv, int hd, int64_t pos0, float scale,
                        int dtype);
