@@ -29,10 +29,10 @@
 // each step's loads. Loading ahead would take the registers of a second workgroup per CU from every call.
 //
 // What bounds it: the MFMAs -- the work counted twice in both products with f32 q, in one with f16 q -- with
-// the softmax's ~11 VALU operations per score beside them from the second wave of each SIMD. Measured
-// (32 / 8 heads of 128): 8192 tokens from 0, f32, 22.3 ms on the vector path and 1.06 ms here (520 of
+// the softmax's ~12 VALU operations per score beside them from the second wave of each SIMD. Measured
+// (32 / 8 heads of 128): 8192 tokens from 0, f32, 22.3 ms on the vector path and 1.03 ms here (530 of
 // the products' own TFLOP/s, twice that of MFMAs); 509 tokens after 3001, 16 / 8 heads, f16, 768 us and
-// 45; one token over 32768 keys, f32, 55 us and 38.6, over 4096, f16, 12.8 us and 11.1.
+// 46.6; one token over 32768 keys, f32, 55 us and 38.2, over 4096, f16, 12.8 us and 11.2.
 #include <algorithm>
 #include <atomic>
 
